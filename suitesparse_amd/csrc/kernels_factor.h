@@ -14,6 +14,11 @@
 
 namespace mxc {
 
+// Row stride of a 64x64 diagonal block and its inverse in LDS: rows start on 16
+// bytes (16-byte reads of a lane's row), and 16 rows 4 banks apart fill the 64
+// banks.
+constexpr int PS = NB + 2;
+
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -300,9 +305,9 @@ __device__ __forceinline__ void pd_tail(const PdArgs &pda, int pd, T *__restrict
     T *S = reinterpret_cast<T *>(smem);
     if (pda.rho > 0) {
         __shared__ double tmp[NB];
-        potrf_block<T, true>(pda.diags[pd], W, S, S + NB * DS, sfail, pda.fail, adiag, pda.rho, pda.rd, tmp);
+        potrf_block<T, true>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, tmp);
     } else {
-        potrf_block<T, false>(pda.diags[pd], W, S, S + NB * DS, sfail, pda.fail, adiag, pda.rho, pda.rd, nullptr);
+        potrf_block<T, false>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, nullptr);
     }
     if (publish) {
         __syncthreads();                    // every wave's stores of L and the inverse are issued
@@ -347,7 +352,7 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     // waves per SIMD either way and keeps two buffers.
     constexpr int NBUF = TS == 128 ? 2 : 1;
     constexpr size_t XY_BYTES = sizeof(T) * NBUF * BK * (TS + LDS_PAD);
-    constexpr size_t PD_BYTES = PD ? sizeof(T) * 2 * NB * DS : 0;
+    constexpr size_t PD_BYTES = PD ? sizeof(T) * 2 * NB * PS : 0;
     // folded TRSM (FP64, 64-wide trailing tiles): the updated block and the
     // next diagonal block's inverse, both k-major like the staged chunks
     constexpr bool CAN_FOLD = PD && MODE == MODE_TRAIL && TS == NB && std::is_same<T, double>::value;
@@ -598,7 +603,7 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
     static_assert(!PD || (MODE == MODE_TRAIL && TS >= 64), "diagonal tails: trailing tiles of 64 or 128");
     // one LDS buffer: the staged halves, reused by the diagonal-block tail
     constexpr size_t H_BYTES = 4 * sizeof(_Float16) * TS * RS;
-    constexpr size_t PD_BYTES = PD ? sizeof(float) * 2 * NB * DS : 0;
+    constexpr size_t PD_BYTES = PD ? sizeof(float) * 2 * NB * PS : 0;
     __shared__ __attribute__((aligned(16))) unsigned char smem[H_BYTES > PD_BYTES ? H_BYTES : PD_BYTES];
     _Float16 *Xh = reinterpret_cast<_Float16 *>(smem);
     _Float16 *Xl = Xh + TS * RS;
@@ -748,27 +753,30 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
 
 // Diagonal block Cholesky + triangular inverse of a 64x64 block (a block
 // narrower than 64 is extended by the identity), one 256-thread workgroup,
-// block-recursive over 16x16 sub-blocks with the 16x16x4 MFMA:
-//   for p = 0..3:  POTRF + inverse of D_pp (one wave, registers)
-//                  panel TRSM  L_tp = A_tp inv(D_pp)'      (MFMA, t > p)
-//                  trailing    A_ij -= L_ip L_jp'          (MFMA, p < j <= i)
-//   inverse:       X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj  (MFMA, block rows i)
-// 18 barriers in all.  The lower factor is written back in place (the strict
-// upper triangle is left alone, as dpotrf leaves it) and inv(L) (zero above
-// the diagonal) goes to the block's inverse slot (ld nb).  A non-positive
-// pivot at column j records col0 + j in *fail (atomic min).
+// over 16-column panels p = 0..3 (panel_elim, potrf_core):
+//   wave 0: rows of panel p, one per lane: POTRF of D_pp and the rows below it
+//           in one elimination (no separate panel TRSM)
+//   wave 1: D_pp again with the 16 identity rows below it: their elimination
+//           leaves inv(D_pp)' (no separate inverse)
+//   waves 2, 3, beside them: panel p-1's other updates (MFMA) and the sums
+//           T_pj = sum_k L_pk X_kj of the inverse's block row p
+//   then, all waves: the update of block column p+1 by panel p (MFMA) and
+//           X_pj = -X_pp T_pj
+// Two barriers per panel.  The lower factor is written back in place (the
+// strict upper triangle is left alone, as dpotrf leaves it) and inv(L) (zero
+// above the diagonal) goes to the block's inverse slot (ld nb).  A
+// non-positive pivot at column j records col0 + j in *fail (atomic min).
 // ---------------------------------------------------------------------------
 
-// 1/sqrt(x) for x > 0: the hardware estimate refined by two Newton steps
-// y <- y + y (1 - x y^2) / 2 (each roughly doubles the correct bits).
+// 1/sqrt(x) for x > 0: the hardware estimate y0 (relative error below 2^-23)
+// refined once to third order, y = y0 (1 + e/2 + 3e^2/8) with e = 1 - x y0^2:
+// the remaining term is below 2^-69, and the chain is four dependent
+// operations where two Newton steps take six (every pivot waits for it).
 __device__ __forceinline__ double rsqrt_nr(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-#pragma unroll
-    for (int it = 0; it < 2; it++) {
-        const double e = fma(-x * y, y, 1.0);
-        y = fma(0.5 * y, e, y);
-    }
-    return y;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    const double ye = y * e;
+    return fma(ye, fma(0.375, e, 0.5), y);
 }
 __device__ __forceinline__ float rsqrt_nr(float x) {
     float y = __builtin_amdgcn_rsqf(x);
@@ -793,14 +801,14 @@ __device__ __forceinline__ float lane_bcast(float v, int k) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
 }
 
-// acc += X * Y' for 16x16 blocks X at S[rx..][cx..], Y at S[ry..][cy..] (row-major, stride DS)
+// acc += X * Y' for 16x16 blocks X at S[rx..][cx..], Y at S[ry..][cy..] (row-major, stride PS)
 template <typename T>
 __device__ __forceinline__ void mma_nt16(const T *S, int rx, int cx, const T *S2, int ry, int cy,
                                          typename MfmaOp<T>::acc_t &acc, int lane) {
 #pragma unroll
     for (int kk = 0; kk < 16; kk += 4) {
-        const T a = S[(rx + (lane & 15)) * DS + cx + kk + (lane >> 4)];
-        const T b = S2[(ry + (lane & 15)) * DS + cy + kk + (lane >> 4)];
+        const T a = S[(rx + (lane & 15)) * PS + cx + kk + (lane >> 4)];
+        const T b = S2[(ry + (lane & 15)) * PS + cy + kk + (lane >> 4)];
         acc = MfmaOp<T>::mma(a, b, acc);
     }
 }
@@ -811,8 +819,8 @@ __device__ __forceinline__ void mma_nn16(const T *S, int rx, int cx, const T *S2
                                          typename MfmaOp<T>::acc_t &acc, int lane) {
 #pragma unroll
     for (int kk = 0; kk < 16; kk += 4) {
-        const T a = S[(rx + (lane & 15)) * DS + cx + kk + (lane >> 4)];
-        const T b = S2[(ry + kk + (lane >> 4)) * DS + cy + (lane & 15)];
+        const T a = S[(rx + (lane & 15)) * PS + cx + kk + (lane >> 4)];
+        const T b = S2[(ry + kk + (lane >> 4)) * PS + cy + (lane & 15)];
         acc = MfmaOp<T>::mma(a, b, acc);
     }
 }
@@ -824,75 +832,148 @@ __device__ __forceinline__ void store16(T *S, int r0, int c0, const typename Mfm
                                         int lane, T alpha, bool accumulate) {
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-        T *q = S + (r0 + MfmaOp<T>::row(lane, v)) * DS + c0 + (lane & 15);
+        T *q = S + (r0 + MfmaOp<T>::row(lane, v)) * PS + c0 + (lane & 15);
         *q = accumulate ? *q + alpha * acc[v] : alpha * acc[v];
     }
 }
 
-// POTRF + inverse of the 16x16 diagonal block at S[R.., R..] (row stride ld)
-// by one wave, lane i < 16 owning row i; the inverse (zero above the diagonal)
-// goes to X in the same layout.  Each pivot costs one reciprocal square root
-// (no divide on the serial path): L_jj = d_jj r_j and L_ij = a_ij r_j with
-// r_j = 1/sqrt(d_jj); the inverse reuses r_j = 1/L_jj.  Returns the first
-// non-positive pivot of the block (16 if none), wave-uniform.  SAFE: *brk is
-// set when a pivot falls to rho * a_jj or below (a_jj the assembled diagonal
-// of A): the block's result is then not used (k_potrf_redo64 refactors it).
-//
-// The inverse is formed column by column (lane c: x_i = r_i (delta_ic -
-// sum_{k<i} L_ik x_k)) with each partial sum updated as soon as x_k is
-// final, the same products in the same order as the row-by-row form.
+// Elimination of a 16-column panel by one wave, a row per lane: lanes 0..15 hold
+// the rows of the diagonal block (their entries above the diagonal are not
+// used), the other lanes rows below it.  On return a[] holds the rows of L:
+// the diagonal block's factor in lanes 0..15 (zero or unused above the
+// diagonal) and A L^-T in the others; an identity row e_q becomes column q of
+// the inverse of the diagonal block.  Each pivot costs one reciprocal square
+// root (no divide on the serial path): L_jj = d_jj r_j and L_ij = a_ij r_j
+// with r_j = 1/sqrt(d_jj).  Returns the first non-positive pivot among the
+// panel's nreal real columns (16 if none), wave-uniform; from that column on
+// the values are not numbers.  SAFE: *brk is set when a pivot falls to its floor or below
+// (floor_l, lane j holds column j's: rho * a_jj, a_jj the assembled diagonal
+// of A): the block's result is then not used (redo_block64 refactors it).
 template <typename T, bool SAFE>
-__device__ __forceinline__ int potrf16_wave(T *S, T *X, int ld, int R, int nb, int lane,
-                                            const double *__restrict__ adiag, int col0, double rho,
-                                            bool *brk) {
-    T a[16], rinv[16];
-#pragma unroll
-    for (int c = 0; c < 16; c++) a[c] = (lane < 16) ? S[(R + lane) * ld + R + c] : (T)0;
-    // pivot floors of the panel's columns (low-precision safeguard), lane j holds column j's
-    T floor_l = 0;
-    if (SAFE && lane < 16 && R + lane < nb) floor_l = (T)(rho * adiag[col0 + R + lane]);
-    // wave-uniform bookkeeping
-    bool low_any = false;   // a pivot at or below its floor
-    int badj = 16;          // first non-positive pivot of the panel
+__device__ __forceinline__ int panel_elim(T (&a)[16], int nreal, T floor_l, bool *brk) {
+    unsigned badm = 0, lowm = 0;    // bit j: pivot j is not positive / at or below its floor
+    T djj = lane_bcast(a[0], 0);
 #pragma unroll
     for (int j = 0; j < 16; j++) {
-        T djj = lane_bcast(a[j], j);
-        const bool real = R + j < nb;
-        if (SAFE) low_any = low_any || (real && djj <= lane_bcast(floor_l, j));
-        const bool bad = !(djj > (T)0);
-        badj = (bad && real && badj == 16) ? j : badj;
-        djj = bad ? (T)1 : djj;
-        const T rj = rsqrt_nr(djj);
-        rinv[j] = rj;
-        const T l = (lane > j) ? a[j] * rj : ((lane == j) ? djj * rj : (T)0);
+        badm |= (unsigned)__ballot(!(djj > (T)0)) & (1u << j);
+        if (SAFE) lowm |= (unsigned)__ballot(djj <= lane_bcast(floor_l, j)) & (1u << j);
+        const T l = a[j] * rsqrt_nr(djj);
         a[j] = l;
+        if (j + 1 < 16) {
+            // the next pivot first: its reciprocal square root then runs beside
+            // the updates of the columns after it
+            a[j + 1] -= l * lane_bcast(l, j + 1);
+            djj = lane_bcast(a[j + 1], j + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        T bl[16];
 #pragma unroll
-        for (int c = j + 1; c < 16; c++) a[c] -= l * lane_bcast(l, c);
+        for (int c = j + 2; c < 16; c++) bl[c] = lane_bcast(l, c);
+#pragma unroll
+        for (int c = j + 2; c < 16; c++) a[c] -= l * bl[c];
     }
-    if (SAFE && low_any) *brk = true;
-    if (lane < 16) {
+    const unsigned realm = nreal >= 16 ? 0xffffu : (1u << nreal) - 1;
+    if (SAFE && (lowm & realm)) *brk = true;
+    badm &= realm;
+    return badm ? __builtin_ctz(badm) : 16;
+}
+
+// Factor and invert the diagonal block of nb columns held in LDS (256
+// threads).  S: the block, NB x PS row-major, its lower triangle (extended by
+// the identity past nb) on entry and L on return; X: its inverse, same layout,
+// the lower triangle's 16x16 blocks on return (blocks above the diagonal are
+// not written).  sfail[0] receives the first failing column (-1 on entry),
+// sfail[1] the breakdown flag (0 on entry).  X's four diagonal 16x16 blocks hold
+// the identity on entry (potrf_init).  The caller synchronizes before;
+// the block and its inverse are complete (and visible) on return.
+template <typename T>
+__device__ __forceinline__ void potrf_init(T *X, int *sfail) {
+    const int tid = threadIdx.x;
 #pragma unroll
-        for (int c = 0; c < 16; c++)
-            if (c <= lane) S[(R + lane) * ld + R + c] = a[c];
+    for (int q = 0; q < 4; q++) {
+        const int e = tid + 256 * q, i = e >> 4, c = e & 15;
+        X[i * PS + (i & ~15) + c] = (i & 15) == c ? (T)1 : (T)0;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    // inverse: lane c < 16 forms column c
-    T x[16], sm[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) sm[i] = (i == lane) ? (T)1 : (T)0;
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-        x[k] = sm[k] * rinv[k];
-#pragma unroll
-        for (int i = k + 1; i < 16; i++) sm[i] -= S[(R + i) * ld + R + k] * x[k];
+    if (tid == 0) {
+        sfail[0] = -1;
+        sfail[1] = 0;
     }
-    if (lane < 16) {
+}
+
+template <typename T, bool SAFE>
+__device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const double *__restrict__ adiag,
+                                           int col0, double rho) {
+    typedef typename MfmaOp<T>::acc_t acc_t;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int np = (nb + 15) >> 4;          // 16-column panels that hold real columns
+    // S(i, j) -= L(i, k) L(j, k)'
+    auto update = [&](int i, int j, int k) {
+        acc_t acc = acc_t{0, 0, 0, 0};
+        // C(m = row in block j, n = row in block i)
+        mma_nt16<T>(S, 16 * j, 16 * k, S, 16 * i, 16 * k, acc, lane);
 #pragma unroll
-        for (int i = 0; i < 16; i++) X[(R + i) * ld + R + lane] = (i >= lane) ? x[i] : (T)0;
+        for (int v = 0; v < 4; v++) S[(16 * i + (lane & 15)) * PS + 16 * j + MfmaOp<T>::row(lane, v)] -= acc[v];
+    };
+    // X(p, j) = -X(p, p) T(p, j), T(p, j) held in X(p, j)
+    auto inv_row = [&](int p, int j) {
+        acc_t acc = acc_t{0, 0, 0, 0};
+        mma_nn16<T>(X, 16 * p, 16 * p, X, 16 * p, 16 * j, acc, lane);
+        wave_sync_lds();                    // the wave's reads of T, before its stores
+        store16<T>(X, 16 * p, 16 * j, acc, lane, (T)-1, false);
+    };
+    for (int p = 0; p < np; p++) {
+        const int R = 16 * p;
+        if (p > 0) {
+            // block column p by panel p-1, and the inverse's block row p-1
+            if (wave < np - p) update(p + wave, p, p - 1);
+            if (wave == 3)
+                for (int j = 0; j < p - 1; j++) inv_row(p - 1, j);
+            __syncthreads();
+        }
+        if (wave < 2) {
+            // wave 0: row R + lane (past the last row: that row again, not stored);
+            // wave 1: the diagonal block's rows, then the identity rows X holds there
+            const bool row = R + lane < NB;
+            const T *ar = (wave == 0 || lane < 16) ? S + min(R + lane, NB - 1) * PS + R
+                                                   : X + (R + (lane & 15)) * PS + R;
+            T a[16];
+#pragma unroll
+            for (int c = 0; c < 16; c++) a[c] = ar[c];
+            T floor_l = 0;
+            if (SAFE && lane < 16 && R + lane < nb) floor_l = (T)(rho * adiag[col0 + R + lane]);
+            bool brk = false;
+            const int badj = panel_elim<T, SAFE>(a, nb - R, floor_l, &brk);
+            if (wave == 0) {
+                if (lane == 0 && badj < 16 && sfail[0] < 0) sfail[0] = R + badj;
+                if (SAFE && lane == 0 && brk) sfail[1] = 1;
+                if (row) {
+#pragma unroll
+                    for (int c = 0; c < 16; c++) S[(R + lane) * PS + R + c] = a[c];
+                }
+            } else if (lane >= 16 && lane < 32) {
+                // lane 16 + q: column q of the inverse
+#pragma unroll
+                for (int c = 0; c < 16; c++) X[(R + c) * PS + R + lane - 16] = a[c];
+            }
+        } else {
+            // waves 2, 3: panel p-1's updates right of block column p, then T(p, j)
+            int q = 0;
+            for (int i = p + 1; p > 0 && i < np; i++)
+                for (int j = p + 1; j <= i; j++)
+                    if ((q++ & 1) == wave - 2) update(i, j, p - 1);
+            for (int j = 0; j < p; j++) {
+                if ((q++ & 1) != wave - 2) continue;
+                acc_t acc = acc_t{0, 0, 0, 0};
+                for (int k = j; k < p; k++) mma_nn16<T>(S, R, 16 * k, X, 16 * k, 16 * j, acc, lane);
+                store16<T>(X, R, 16 * j, acc, lane, (T)1, false);
+            }
+        }
+        __syncthreads();
     }
-    return badj;
+    if (np > 1) {
+        if (wave < np - 1) inv_row(np - 1, wave);
+        __syncthreads();
+    }
 }
 
 // SAFE (rho > 0, low-precision factor): a pivot d_jj <= rho * a_jj (a_jj the
@@ -903,7 +984,7 @@ __device__ __forceinline__ int potrf16_wave(T *S, T *X, int ld, int R, int nb, i
 // <= 0 is reported as the failing column.
 //
 // potrf_block: the whole workgroup (256 threads) factors diagonal block t in
-// LDS (S: the block, X: its inverse, both NB x DS row-major and contiguous;
+// LDS (S: the block, X: its inverse, both NB x PS row-major and contiguous;
 // sfail: two shared ints, the first failing column and the breakdown flag;
 // tmp: NB shared doubles for the redo) and writes L_tt and the inverse back
 // to W.
@@ -911,126 +992,42 @@ template <typename T, bool SAFE>
 __device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W, T *S, T *X, int *sfail,
                                             int *__restrict__ fail, const double *__restrict__ adiag,
                                             double rho, const Redo &rd, double *tmp) {
-    typedef typename MfmaOp<T>::acc_t acc_t;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x;
     const int nb = t.nb;
-    const int np = (nb + 15) >> 4;          // 16-column panels that hold real columns
+    const int i = tid & (NB - 1), c0 = tid >> 6;
     {
-        // all 16 loads of a thread in flight at once, then the LDS stores
+        // all 16 loads of a thread in flight at once (unconditional, from inside the
+        // block: a predicated load is a branch each), then the LDS stores
         T v[16];
-        const int i = tid & (NB - 1), c0 = tid >> 6;
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             const int c = c0 + 4 * q;
-            v[q] = (i < nb && c < nb && c <= i) ? W[t.off + i + (long long)c * t.ld] : (T)0;
+            v[q] = W[t.off + min(i, nb - 1) + (long long)min(c, nb - 1) * t.ld];
         }
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             const int c = c0 + 4 * q;
-            S[i * DS + c] = (i >= nb && i == c) ? (T)1 : v[q];
-            X[i * DS + c] = 0;
+            S[i * PS + c] = (i < nb && c < nb) ? (c <= i ? v[q] : (T)0) : (i == c ? (T)1 : (T)0);
         }
     }
-    if (tid == 0) {
-        sfail[0] = -1;
-        sfail[1] = 0;
-    }
+    potrf_init(X, sfail);
     __syncthreads();
-
-    // Right-looking over 16-column panels, one panel of look-ahead: after the
-    // TRSM of panel p, wave 0 updates only the next diagonal block and factors
-    // it at once, while waves 1..3 apply panel p's other updates and form block
-    // row p of the inverse, whose inputs are final by then:
-    //   L_ii, X_ii = potrf16_wave(S_ii);   L_ip = S_ip X_pp';
-    //   S_ij -= L_ip L_jp' (p < j <= i);   X_pj = -X_pp sum_{k=j}^{p-1} L_pk X_kj (j < p).
-    if (wave == 0) {
-        bool brk = false;
-        const int badj = potrf16_wave<T, SAFE>(S, X, DS, 0, nb, lane, adiag, t.col0, rho, &brk);
-        if (lane == 0 && badj < 16 && sfail[0] < 0) sfail[0] = badj;
-        if (SAFE && lane == 0 && brk) sfail[1] = 1;
-    }
-    __syncthreads();
-    for (int p = 0; p < np; p++) {
-        const int R = 16 * p;
-        // (1) panel TRSM: rows below, 16-row tiles p+1..np-1, one wave each
-        if (wave < np - 1 - p) {
-            const int rt = 16 * (p + 1 + wave);
-            acc_t acc = acc_t{0, 0, 0, 0};
-            // C(m = row of inv, n = panel row) = sum_k X(m, k) A(n, k)  ->  L(n, m)
-            mma_nt16<T>(X, R, R, S, rt, R, acc, lane);
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                S[(rt + (lane & 15)) * DS + R + MfmaOp<T>::row(lane, v)] = acc[v];
-        }
-        __syncthreads();
-        if (wave == 0) {
-            // (2a) the next diagonal block: its update by panel p, then its POTRF
-            if (p + 1 < np) {
-                const int Q = R + 16;
-                acc_t acc = acc_t{0, 0, 0, 0};
-                mma_nt16<T>(S, Q, R, S, Q, R, acc, lane);
-#pragma unroll
-                for (int v = 0; v < 4; v++) S[(Q + (lane & 15)) * DS + Q + MfmaOp<T>::row(lane, v)] -= acc[v];
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                bool brk = false;
-                const int badj = potrf16_wave<T, SAFE>(S, X, DS, Q, nb, lane, adiag, t.col0, rho, &brk);
-                if (lane == 0 && badj < 16 && sfail[0] < 0) sfail[0] = Q + badj;
-                if (SAFE && lane == 0 && brk) sfail[1] = 1;
-            }
-        } else {
-            // (2b) waves 1..3, round robin: panel p's other updates, then block row p of the inverse
-            int q = 0;
-            for (int i = p + 1; i < np; i++)
-                for (int j = p + 1; j <= i; j++) {
-                    if (i == p + 1 && j == p + 1) continue;
-                    if ((q++ % 3) != wave - 1) continue;
-                    acc_t acc = acc_t{0, 0, 0, 0};
-                    // C(m = row in block j, n = row in block i) = sum_k L_jp(m,k) L_ip(n,k)
-                    mma_nt16<T>(S, 16 * j, R, S, 16 * i, R, acc, lane);
-#pragma unroll
-                    for (int v = 0; v < 4; v++) {
-                        T *dst = S + (16 * i + (lane & 15)) * DS + 16 * j + MfmaOp<T>::row(lane, v);
-                        *dst -= acc[v];
-                    }
-                }
-            for (int j = 0; j < p; j++) {
-                if ((q++ % 3) != wave - 1) continue;
-                acc_t tacc = acc_t{0, 0, 0, 0};
-                for (int k = j; k < p; k++) mma_nn16<T>(S, R, 16 * k, X, 16 * k, 16 * j, tacc, lane);
-                // stage T = sum_k L_pk X_kj in X's (still zero) block (p, j), then X_pj = -X_pp T
-                store16<T>(X, R, 16 * j, tacc, lane, (T)1, false);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-                acc_t acc = acc_t{0, 0, 0, 0};
-                mma_nn16<T>(X, R, R, X, R, 16 * j, acc, lane);
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-                __builtin_amdgcn_wave_barrier();
-                store16<T>(X, R, 16 * j, acc, lane, (T)-1, false);
-            }
-        }
-        __syncthreads();
-    }
+    potrf_core<T, SAFE>(S, X, sfail, nb, adiag, t.col0, rho);
     if (SAFE && sfail[1]) {
         // breakdown: the block again from W, in FP64, in the LDS of S and X
-        static_assert(!SAFE || sizeof(T) * 2 * NB * DS >= sizeof(double) * NB * (NB + 1),
+        static_assert(!SAFE || sizeof(T) * 2 * NB * PS >= sizeof(double) * NB * (NB + 1),
                       "the FP64 redo needs the LDS of S and X");
         redo_block64<T>(t, W, reinterpret_cast<double *>(S), tmp, sfail, tid, 256, rd, fail,
                         [] { __syncthreads(); });
         return;
     }
     if (tid == 0 && sfail[0] >= 0) atomicMin(fail, t.col0 + sfail[0]);
-    {
-        const int i = tid & (NB - 1), c0 = tid >> 6;
 #pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const int c = c0 + 4 * q;
-            if (i < nb && c < nb) {
-                if (c <= i) W[t.off + i + (long long)c * t.ld] = S[i * DS + c];
-                W[t.winv + i + (long long)c * nb] = (c <= i) ? X[i * DS + c] : (T)0;
-            }
+    for (int q = 0; q < 16; q++) {
+        const int c = c0 + 4 * q;
+        if (i < nb && c < nb) {
+            if (c <= i) W[t.off + i + (long long)c * t.ld] = S[i * PS + c];
+            W[t.winv + i + (long long)c * nb] = (c <= i) ? X[i * PS + c] : (T)0;
         }
     }
 }
@@ -1039,65 +1036,54 @@ template <typename T, bool SAFE>
 __global__ __launch_bounds__(256) void k_potrf_diag(const DiagTask *__restrict__ tasks,
                                                     T *__restrict__ W, int *__restrict__ fail,
                                                     const double *__restrict__ adiag, double rho, Redo rd) {
-    __shared__ __attribute__((aligned(16))) T SX[2 * NB * DS];   // the block and its inverse, row-major
+    __shared__ __attribute__((aligned(16))) T SX[2 * NB * PS];   // the block and its inverse, row-major
     __shared__ int sfail[2];
     __shared__ double tmp[SAFE ? NB : 1];
-    potrf_block<T, SAFE>(tasks[blockIdx.x], W, SX, SX + NB * DS, sfail, fail, adiag, rho, rd, tmp);
+    potrf_block<T, SAFE>(tasks[blockIdx.x], W, SX, SX + NB * PS, sfail, fail, adiag, rho, rd, tmp);
 }
 
 
 // Diagonal blocks of at most 16 columns (the many tiny supernodes of the
 // lower etree levels): one wave per block, four blocks per workgroup, the
-// same POTRF + inverse as panel 0 of k_potrf_diag.
+// block and its inverse from one elimination (panel_elim).
 template <typename T, bool SAFE>
 __global__ __launch_bounds__(256) void k_potrf_small(const DiagTask *__restrict__ tasks, int ntask,
                                                      T *__restrict__ W, int *__restrict__ fail,
                                                      const double *__restrict__ adiag, double rho, Redo rd) {
-    constexpr int SS = 17;
-    __shared__ T S[4][16 * SS];
-    __shared__ T X[4][16 * SS];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int ti = blockIdx.x * 4 + w;
     if (ti >= ntask) return;
     const DiagTask t = tasks[ti];
     const int nb = t.nb;
-    T *Sw = S[w], *Xw = X[w];
-    if (lane < 16) {
-        T v[16];
+    // lanes 0..15: the block's rows (extended by the identity), lanes 16..31: identity rows
+    T a[16];
 #pragma unroll
-        for (int c = 0; c < 16; c++)
-            v[c] = (lane < nb && c <= lane) ? W[t.off + lane + (long long)c * t.ld] : (T)0;
-#pragma unroll
-        for (int c = 0; c < 16; c++) Sw[lane * SS + c] = (lane >= nb && lane == c) ? (T)1 : v[c];
+    for (int c = 0; c < 16; c++) {
+        // (loads from inside the block, unconditional: a predicated load is a branch each)
+        const T v = W[t.off + min(lane, nb - 1) + (long long)min(c, nb - 1) * t.ld];
+        a[c] = (lane < nb && c <= lane) ? v : ((lane < 32 && (lane & 15) == c) ? (T)1 : (T)0);
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    T floor_l = 0;
+    if (SAFE && lane < nb) floor_l = (T)(rho * adiag[t.col0 + lane]);
     bool brk = false;
-    const int badj = potrf16_wave<T, SAFE>(Sw, Xw, SS, 0, nb, lane, adiag, t.col0, rho, &brk);
+    const int badj = panel_elim<T, SAFE>(a, nb, floor_l, &brk);
     if (SAFE && brk) {
         // breakdown: leave the assembled block in W for the FP64 redo
         if (lane == 0) redo_push(rd, t);
         return;
     }
     if (lane == 0 && badj < nb) atomicMin(fail, t.col0 + badj);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if (lane < nb) {
+    // L by rows; lane 16 + q holds column q of the inverse
 #pragma unroll
-        for (int c = 0; c < 16; c++) {
-            if (c < nb) {
-                if (c <= lane) W[t.off + lane + (long long)c * t.ld] = Sw[lane * SS + c];
-                W[t.winv + lane + (long long)c * nb] = (c <= lane) ? Xw[lane * SS + c] : (T)0;
-            }
-        }
+    for (int c = 0; c < 16; c++) {
+        if (lane < nb && c <= lane) W[t.off + lane + (long long)c * t.ld] = a[c];
+        if (lane >= 16 && lane - 16 < nb && c < nb) W[t.winv + c + (long long)(lane - 16) * nb] = a[c];
     }
 }
 
 // Diagonal blocks of at most TINY_DIAG columns (the bottom levels of a forest:
 // mostly one to five columns): one lane factors and inverts a whole block, with
-// potrf16_wave's arithmetic: pivot d_jj (when SAFE, a pivot at or below
+// panel_elim's arithmetic: pivot d_jj (when SAFE, a pivot at or below
 // rho a_jj sends the block to the FP64 redo queue), a non-positive pivot
 // reported and replaced by 1, r_j = 1/sqrt(d_jj), L_jj = d_jj r_j,
 // L_ij = a_ij r_j, the inverse by forward substitution with r_j.
@@ -1248,7 +1234,7 @@ __global__ __launch_bounds__(256) void k_trsm_tiny(const UpdDesc *__restrict__ d
 // of X), then S[rel(i)][rel(j)] -= C(i, j) for i >= j by LDS atomics, rel the
 // block rows' positions among the supernode's rows.  Factorization, by wave 0:
 // right-looking over the nscol columns with lane r owning row r of the panel,
-// potrf16_wave's pivot arithmetic (r_j = 1/sqrt(d_jj), L_jj = d_jj r_j,
+// panel_elim's pivot arithmetic (r_j = 1/sqrt(d_jj), L_jj = d_jj r_j,
 // L_rj = a_rj r_j, a non-positive pivot reported and replaced by 1) applied
 // to the rows below the diagonal block as well, which makes the TRSM part of
 // the same pass.  The inverse of the diagonal block is formed as potrf16_wave
