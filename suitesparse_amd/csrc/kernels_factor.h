@@ -373,6 +373,41 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wr = TS <= 32 ? 0 : (wave & 1), wc = TS <= 32 ? 0 : (wave >> 1);
 
+    // thread t stages row r = t % TS of chunk rows k = t/TS + KG*q, q < PER.  The
+    // loads are unconditional (rows and k clamped into the block, a predicated
+    // load is a branch each): rows past the block's edge give entries of C that
+    // are not stored, and columns past K are staged as zeros.  k is the same for
+    // a whole wave in the four-wave tiles.
+    const T *__restrict__ Xp = W + d.x_off;
+    const T *__restrict__ Yp = W + d.y_off;
+    const int r = tid % TS;
+    const int kq = TS >= 64 ? __builtin_amdgcn_readfirstlane(tid / TS) : tid / TS;
+    const unsigned yo = (unsigned)min(i0 + r, d.M - 1) * (unsigned)sizeof(T);
+    const unsigned xo = (unsigned)min(j0 + r, d.N - 1) * (unsigned)sizeof(T);
+    auto at = [](const T *p, unsigned o) {
+        return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + o);
+    };
+    T ry[PER], rx[PER];
+    auto fetch = [&](int k0) {
+        if (k0 + BK <= d.K) {
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                ry[q] = at(Yp + (long long)(k0 + kq + KG * q) * d.ldy, yo);
+                rx[q] = at(Xp + (long long)(k0 + kq + KG * q) * d.ldx, xo);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                const int gk = min(k0 + kq + KG * q, d.K - 1);
+                const bool kin = k0 + kq + KG * q < d.K;
+                const T y = at(Yp + (long long)gk * d.ldy, yo), x = at(Xp + (long long)gk * d.ldx, xo);
+                ry[q] = kin ? y : (T)0;
+                rx[q] = kin ? x : (T)0;
+            }
+        }
+    };
+    fetch(0);                                   // in flight during the search below
+
     if (MODE == MODE_SCATTER) {
         for (int e = tid; e < 2 * TS; e += NT) {
             if (e < TS) {
@@ -405,24 +440,6 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
 #pragma unroll
         for (int b = 0; b < MB; b++) acc[a][b] = acc_t{0, 0, 0, 0};
 
-    const T *__restrict__ Xp = W + d.x_off;
-    const T *__restrict__ Yp = W + d.y_off;
-    // thread t stages row r = t % TS of chunk rows k = t/TS + KG*q, q < PER
-    const int r = tid % TS, kq = tid / TS;
-    const bool rowy = (i0 + r) < d.M, rowx = (j0 + r) < d.N;
-    const T *yrow = Yp + (i0 + r);
-    const T *xrow = Xp + (j0 + r);
-    T ry[PER], rx[PER];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            const int gk = k0 + kq + KG * q;
-            const bool kin = gk < d.K;
-            ry[q] = (kin && rowy) ? yrow[(long long)gk * d.ldy] : (T)0;
-            rx[q] = (kin && rowx) ? xrow[(long long)gk * d.ldx] : (T)0;
-        }
-    };
-    fetch(0);
     int buf = 0;
     for (int k0 = 0; k0 < d.K; k0 += BK) {
         if (NBUF == 1 && k0 > 0) __syncthreads();   // the previous chunk's reads are done
@@ -433,17 +450,27 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
         }
         __syncthreads();
         if (k0 + BK < d.K) fetch(k0 + BK);      // next chunk in flight during the MFMAs
+        // operands one step ahead: their LDS latency passes under the MFMAs
+        // (with the unconditional loads, one 64-wide FP64 launch over 6000 x 5600,
+        // K = 384: 55.5 -> 60.5 TFLOP/s; a chunk alone on its CU 2,190 -> 1,920
+        // cycles, of which the MFMAs take 1,024)
+        T xa[2][MB], yb[2][MB];
+        auto operands = [&](int kk, T (&x)[MB], T (&y)[MB]) {
+#pragma unroll
+            for (int m = 0; m < MB; m++) x[m] = Xs[buf][kk + (lane >> 4)][wc * WB + m * 16 + (lane & 15)];
+#pragma unroll
+            for (int n = 0; n < MB; n++) y[n] = Ys[buf][kk + (lane >> 4)][wr * WB + n * 16 + (lane & 15)];
+        };
+        operands(0, xa[0], yb[0]);
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 4) {
-            T xa[MB], yb[MB];
-#pragma unroll
-            for (int m = 0; m < MB; m++) xa[m] = Xs[buf][kk + (lane >> 4)][wc * WB + m * 16 + (lane & 15)];
-#pragma unroll
-            for (int n = 0; n < MB; n++) yb[n] = Ys[buf][kk + (lane >> 4)][wr * WB + n * 16 + (lane & 15)];
+            const int c = (kk >> 2) & 1;
+            if (kk + 4 < BK) operands(kk + 4, xa[c ^ 1], yb[c ^ 1]);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int m = 0; m < MB; m++)
 #pragma unroll
-                for (int n = 0; n < MB; n++) acc[m][n] = MfmaOp<T>::mma(xa[m], yb[n], acc[m][n]);
+                for (int n = 0; n < MB; n++) acc[m][n] = MfmaOp<T>::mma(xa[c][m], yb[c][n], acc[m][n]);
         }
         if constexpr (NBUF == 2) buf ^= 1;
     }
@@ -553,8 +580,8 @@ __global__ __launch_bounds__(TS <= 32 ? 64 : 256, TS == 128 ? 2 : 1) void k_tile
 
 // The tiles of a launch on a grid of at most a few workgroups per CU (a
 // multiple of 8, so a workgroup's tiles keep its XCD): the second-stream
-// trailing update leaves room on every CU for the diagonal factorizations
-// of the main stream, which otherwise wait until the whole launch drains.
+// trailing update under MXC_OPT_T2_GRID, which leaves room on every CU for
+// the main stream's launches.
 template <typename T, int MODE, int TS>
 __global__ __launch_bounds__(256, 1) void k_tile_grid(const UpdDesc *__restrict__ descs,
                                                       const Tile *__restrict__ tiles, T *__restrict__ W,
@@ -655,22 +682,29 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
     __syncthreads();
 
     // staging: thread t holds row r = t % TS, k in [kq * PER, kq * PER + PER) of a chunk
-    const int r = tid % TS, kq = tid / TS;
-    const bool rowy = (i0 + r) < d.M, rowx = (j0 + r) < d.N;
-    const unsigned *yrow = Lh + d.y_off + (i0 + r);
-    const unsigned *xrow = Lh + d.x_off + (j0 + r);
+    // (unconditional loads, rows and k clamped; columns past K staged as zeros)
+    const int r = tid % TS, kq = __builtin_amdgcn_readfirstlane(tid / TS);
+    const int yr = min(i0 + r, d.M - 1), xr = min(j0 + r, d.N - 1);
+    const unsigned *Yp = Lh + d.y_off, *Xp = Lh + d.x_off;
     unsigned ry[PER], rx[PER];
     auto fetch = [&](int k0) {
 #pragma unroll
         for (int q = 0; q < PER; q++) {
-            const int gk = k0 + kq * PER + q;
-            const bool kin = gk < d.K;
-            ry[q] = (kin && rowy) ? yrow[(long long)gk * d.ldy] : 0u;
-            rx[q] = (kin && rowx) ? xrow[(long long)gk * d.ldx] : 0u;
+            const int gk = min(k0 + kq * PER + q, d.K - 1);
+            ry[q] = Yp[(long long)gk * d.ldy + yr];
+            rx[q] = Xp[(long long)gk * d.ldx + xr];
         }
     };
     auto half_of = [](unsigned u) { return __builtin_bit_cast(_Float16, (unsigned short)(u & 0xffffu)); };
-    auto stage = [&]() {
+    auto stage = [&](int k0) {
+        if (k0 + BKH > d.K) {
+#pragma unroll
+            for (int q = 0; q < PER; q++) {
+                const bool kin = k0 + kq * PER + q < d.K;
+                ry[q] = kin ? ry[q] : 0u;
+                rx[q] = kin ? rx[q] : 0u;
+            }
+        }
 #pragma unroll
         for (int h = 0; h < PER; h += 8) {
             half8_t yh, yl, xh, xl;
@@ -699,7 +733,7 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
     const int ko = 8 * (lane >> 4);
     for (int k0 = 0; k0 < d.K; k0 += BKH) {
         __syncthreads();                         // the previous chunk's reads are done
-        stage();
+        stage(k0);
         __syncthreads();
         if (k0 + BKH < d.K) fetch(k0 + BKH);     // next chunk in flight during the MFMAs
         half8_t xh[MB], xl[MB], yh[MB], yl[MB];
@@ -1057,9 +1091,11 @@ __global__ __launch_bounds__(256) void k_potrf_diag(const DiagTask *__restrict__
 // after that.
 //
 // What bounds it: the chain of diagonal blocks (hand-off, inverse load, TRSM,
-// product, potrf_core per 64 columns); the launches per step that this
-// replaces (TRSM, then trailing tiles with the next block's factorization as a
-// tail) cost a launch and a reload of the block from HBM each.
+// product, potrf_core: 17 us per 64 columns, of which potrf_core 8); the
+// launches per step that this replaces (TRSM, then trailing tiles with the next
+// block's factorization as a tail) took 50 us per step at 64^3.  64 rows per
+// workgroup: a panel of the largest supernodes (14,600 rows) is then 229
+// workgroups, one per CU, and small ones still spread.
 //
 // Hand-off: as in the chained sweeps (kernels_solve.h), published blocks and
 // flags are stored and loaded by device-scope atomics, performed at the device
@@ -1099,23 +1135,24 @@ __device__ __forceinline__ void panel_publish(int *flag) {
     if (threadIdx.x == 0) dev_store(flag, 1);
 }
 
+// Row stride of the panel workgroups' two 64 x 64 buffers: two workgroups of
+// doubles fit a CU's 160 KB.
+constexpr int PANEL_LD = NB + 4;
+
 template <typename T, bool SAFE, bool DIAG>
 __device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W, const int *__restrict__ Ls,
                                            unsigned *__restrict__ Lh, const double *__restrict__ adiag,
                                            int *__restrict__ fail, double rho, const Redo &rd,
                                            int *__restrict__ ready, int *__restrict__ abort, T *smem) {
     typedef typename MfmaOp<T>::acc_t acc_t;
-    constexpr int LD = NB + LDS_PAD;
+    constexpr int LD = PANEL_LD;
     T(*Am)[LD] = reinterpret_cast<T(*)[LD]>(smem);              // Am[j][i]: the block of A, then of L
     T(*Im)[LD] = reinterpret_cast<T(*)[LD]>(smem + NB * LD);    // Im[k][j] = inv(j, k)
-    T(*Xs)[LD] = Im;                                            // staged chunks (before Im is loaded)
-    T(*Ys)[LD] = reinterpret_cast<T(*)[LD]>(smem + (NB + BK) * LD);
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);     // (a scalar: offsets by w need no vector registers)
     const int l15 = lane & 15, l4 = lane >> 4;
-    const int r = lane, kq = w;                                 // staging: row r, k = kq + 4 q
     const int nsteps = DIAG ? t.blk : (t.ncols + NB - 1) / NB;
     T *Wr = W + t.lx + t.r0;                                    // the workgroup's rows, column 0
-    const T *yrow = Wr + min(r, t.nr - 1);
     auto own = [](const T *p) { return DIAG ? dev_load(p) : *p; };
     int ex = 0;                                                 // FP32: the split-FP16 scale of row 16 w + l15
     const bool h16 = std::is_same<T, float>::value && Lh;
@@ -1123,74 +1160,88 @@ __device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W
 
     // the diagonal block: lower 16x16 blocks q = w, w + 4, w + 8 of the column-by-column list
     constexpr int NDB = DIAG ? 3 : 1;
-    const int dbi[3] = {w, w == 3 ? 2 : w + 1, w == 0 ? 3 : 3}, dbj[3] = {0, w == 3 ? 2 : 1, w == 0 ? 2 : 3};
-    acc_t accD[NDB];
-    T dv[NDB][4];
+    const int dbi[3] = {w, w == 3 ? 2 : w + 1, 3}, dbj[3] = {0, w == 3 ? 2 : 1, w == 0 ? 2 : 3};
     const int nd = w < 2 ? 3 : 2;
-    if constexpr (DIAG) {
-        const T *Wd = Wr + (long long)t.r0 * t.ld;
+    acc_t accD[NDB];
 #pragma unroll
-        for (int q = 0; q < 3; q++) {
-            accD[q] = acc_t{0, 0, 0, 0};
+    for (int q = 0; q < NDB; q++) accD[q] = acc_t{0, 0, 0, 0};
+    // its sum over one more block of the workgroup's rows, held in Am
+    auto product = [&]() {
 #pragma unroll
-            for (int v = 0; v < 4; v++)
-                dv[q][v] = Wd[min(16 * dbi[q] + l15, t.nr - 1) +
-                              (long long)min(16 * dbj[q] + MfmaOp<T>::row(lane, v), t.nr - 1) * t.ld];
-        }
-    }
+        for (int q = 0; q < NDB; q++)
+            if (q < nd) {
+#pragma unroll
+                for (int kk = 0; kk < NB; kk += 4)
+                    accD[q] = MfmaOp<T>::mma(Am[kk + l4][16 * dbj[q] + l15], Am[kk + l4][16 * dbi[q] + l15], accD[q]);
+            }
+    };
 
     for (int s = 0; s < nsteps; s++) {
         const int nbs = min(NB, t.ncols - s * NB);
         T *Ws = Wr + (long long)s * NB * t.ld;                  // the block's column 0
-        // C on 2 x 2 waves of 2 x 2 MFMA blocks; the block's own values beside it
+        if (DIAG && s > 0) {
+            product();
+            // the last block's device-scope stores are complete (every thread's,
+            // with the barrier) before the loads of the workgroup's own rows below:
+            // a device-scope load may pass a store of another wave in flight
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();                                    // and Am is staged into below
+        }
+        // C on 2 x 2 waves of 2 x 2 MFMA blocks
         const int wr = w & 1, wc = w >> 1;
         acc_t acc[2][2];
-        T av[2][2][4];
 #pragma unroll
         for (int m = 0; m < 2; m++)
 #pragma unroll
-            for (int n = 0; n < 2; n++) {
-                acc[m][n] = acc_t{0, 0, 0, 0};
+            for (int n = 0; n < 2; n++) acc[m][n] = acc_t{0, 0, 0, 0};
+        constexpr int CK = 32, PER = CK / 4;
+        T g[16];                                                // loads in flight: X and Y of a stage, or A
+        auto fetch_a = [&]() {
 #pragma unroll
-                for (int v = 0; v < 4; v++)
-                    av[m][n][v] = Ws[min(32 * wr + 16 * n + l15, t.nr - 1) +
-                                     (long long)min(32 * wc + 16 * m + MfmaOp<T>::row(lane, v), nbs - 1) * t.ld];
-            }
+            for (int e = 0; e < 16; e++)
+                g[e] = Ws[min(32 * wr + 16 * ((e >> 2) & 1) + l15, t.nr - 1) +
+                          (long long)min(32 * wc + 16 * (e >> 3) + MfmaOp<T>::row(lane, e & 3), nbs - 1) * t.ld];
+        };
+        if (s == 0) fetch_a();
         if (s > 0) {
             panel_wait(ready + t.flag + 2 * s, abort);
-            const T *xrow = W + t.lx + s * NB + min(r, nbs - 1);
-            T rx[4], ry[4];
+            // 32 columns per stage (in Am and Im, free until the sums are complete):
+            // its 32 products per wave cover the latency of the next stage's loads
+            const T *xrow = W + t.lx + s * NB, *yrow = Wr;
+            const int xr = min(lane, nbs - 1), yr = min(lane, t.nr - 1);
             auto fetch = [&](int k0) {
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    const long long o = (long long)(k0 + kq + 4 * q) * t.ld;
-                    rx[q] = dev_load(xrow + o);
-                    ry[q] = own(yrow + o);
+                for (int q = 0; q < PER; q++) {
+                    const long long o = (long long)(k0 + w + 4 * q) * t.ld;
+                    g[q] = dev_load(xrow + o + xr);
+                    g[PER + q] = own(yrow + o + yr);
                 }
             };
             fetch(0);
-            for (int k0 = 0; k0 < s * NB; k0 += BK) {
-                __syncthreads();                                // the previous chunk's reads are done
+            for (int k0 = 0; k0 < s * NB; k0 += CK) {
+                if (k0 > 0) __syncthreads();                    // the previous stage's reads are done
 #pragma unroll
-                for (int q = 0; q < 4; q++) {
-                    Xs[kq + 4 * q][r] = rx[q];
-                    Ys[kq + 4 * q][r] = ry[q];
+                for (int q = 0; q < PER; q++) {
+                    Im[w + 4 * q][lane] = g[q];
+                    Am[w + 4 * q][lane] = g[PER + q];
                 }
                 __syncthreads();
-                if (k0 + BK < s * NB) fetch(k0 + BK);
+                if (k0 + CK < s * NB) fetch(k0 + CK);
+                else fetch_a();
 #pragma unroll
-                for (int kk = 0; kk < BK; kk += 4) {
+                for (int kk = 0; kk < CK; kk += 4) {
                     T xa[2], yb[2];
 #pragma unroll
-                    for (int m = 0; m < 2; m++) xa[m] = Xs[kk + l4][32 * wc + 16 * m + l15];
+                    for (int m = 0; m < 2; m++) xa[m] = Im[kk + l4][32 * wc + 16 * m + l15];
 #pragma unroll
-                    for (int n = 0; n < 2; n++) yb[n] = Ys[kk + l4][32 * wr + 16 * n + l15];
+                    for (int n = 0; n < 2; n++) yb[n] = Am[kk + l4][32 * wr + 16 * n + l15];
 #pragma unroll
                     for (int m = 0; m < 2; m++)
 #pragma unroll
                         for (int n = 0; n < 2; n++) acc[m][n] = MfmaOp<T>::mma(xa[m], yb[n], acc[m][n]);
                 }
             }
+            __syncthreads();                                    // the staged columns' reads are done
         }
 #pragma unroll
         for (int m = 0; m < 2; m++)
@@ -1199,7 +1250,7 @@ __device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
                     const int j = 32 * wc + 16 * m + MfmaOp<T>::row(lane, v);
-                    Am[j][32 * wr + 16 * n + l15] = j < nbs ? av[m][n][v] - acc[m][n][v] : (T)0;
+                    Am[j][32 * wr + 16 * n + l15] = j < nbs ? g[8 * m + 4 * n + v] - acc[m][n][v] : (T)0;
                 }
         // the inverse of block s
         panel_wait(ready + t.flag + 2 * s + 1, abort);
@@ -1207,7 +1258,6 @@ __device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W
         T iv[16];
 #pragma unroll
         for (int q = 0; q < 16; q++) iv[q] = dev_load(inv + min(lane, nbs - 1) + min(w + 4 * q, nbs - 1) * nbs);
-        __syncthreads();                                        // the staged chunks' reads are done
 #pragma unroll
         for (int q = 0; q < 16; q++) Im[w + 4 * q][lane] = (lane < nbs && w + 4 * q < nbs) ? iv[q] : (T)0;
         __syncthreads();
@@ -1241,18 +1291,8 @@ __device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W
             for (int jb = 0; jb < 4; jb++)
 #pragma unroll
                 for (int v = 0; v < 4; v++) Am[16 * jb + MfmaOp<T>::row(lane, v)][i] = l[jb][v];
-            if (s == nsteps - 1) panel_publish(ready + t.flag + 2 * t.blk);
-            else __syncthreads();
-#pragma unroll
-            for (int q = 0; q < 3; q++)
-                if (q < nd) {
-#pragma unroll
-                    for (int kk = 0; kk < NB; kk += 4)
-                        accD[q] = MfmaOp<T>::mma(Am[kk + l4][16 * dbj[q] + l15], Am[kk + l4][16 * dbi[q] + l15],
-                                                 accD[q]);
-                }
         }
-        __syncthreads();                                        // Am and Im are rewritten by the next step
+        __syncthreads();                                        // Am is complete, Im free
     }
 
     if constexpr (DIAG) {
@@ -1260,6 +1300,17 @@ __device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W
         T *S = smem, *X = smem + NB * PS;
         T *Wd = Wr + (long long)t.r0 * t.ld;
         const int nb = t.nr;
+        T dv[3][4];
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                dv[q][v] = Wd[min(16 * dbi[q] + l15, nb - 1) +
+                              (long long)min(16 * dbj[q] + MfmaOp<T>::row(lane, v), nb - 1) * t.ld];
+        if (nsteps > 0) {
+            product();
+            __syncthreads();                                    // Am's reads are done (S takes its place)
+        }
 #pragma unroll
         for (int q = 0; q < 3; q++) {
             if (q >= nd) break;
@@ -1275,7 +1326,8 @@ __device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W
             }
         }
         potrf_init(X, sfail);
-        __syncthreads();
+        // (the rows' stores have had the product's time to complete)
+        panel_publish(ready + t.flag + 2 * t.blk);
         const int col0 = t.col0 + t.blk * NB;
         potrf_core<T, SAFE>(S, X, sfail, nb, adiag, col0, rho);
         int *flag = ready + t.flag + 2 * t.blk + 1;
@@ -1311,9 +1363,12 @@ __global__ __launch_bounds__(256, 2) void k_panel(const PanelTask *__restrict__ 
                                                   const double *__restrict__ adiag, int *__restrict__ fail,
                                                   double rho, Redo rd, int *__restrict__ ready,
                                                   int *__restrict__ abort) {
-    __shared__ __attribute__((aligned(16))) T smem[2 * NB * (NB + LDS_PAD)];
-    static_assert(PS <= NB + LDS_PAD, "the diagonal block and its inverse fit the staging buffers");
+    __shared__ __attribute__((aligned(16))) T smem[2 * NB * PANEL_LD];
+    static_assert(PS <= PANEL_LD, "the diagonal block and its inverse fit the staging buffers");
     const PanelTask t = tasks[blockIdx.x];
+    // the chain of diagonal blocks goes ahead of the second stream's trailing
+    // tiles on its CUs (wave priority: 80^3 27-point FP64 54.0 -> 53.6 ms)
+    if (t.blk >= 0) __builtin_amdgcn_s_setprio(3);
     if (t.blk >= 0) panel_rows<T, SAFE, true>(t, W, Ls, Lh, adiag, fail, rho, rd, ready, abort, smem);
     else panel_rows<T, SAFE, false>(t, W, Ls, Lh, adiag, fail, rho, rd, ready, abort, smem);
 }

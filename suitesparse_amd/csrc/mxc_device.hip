@@ -245,7 +245,7 @@ struct mxc_factor {
     int64_t panel_flags = 0;             // first of the panel factorizations' flags in d_ready
     PanelTask *d_panel = nullptr;
     bool merge_t2 = true;                // FP64: fold second-stream updates into later trailing launches
-    int t2_per_cu = 3;                   // FP64 second-stream trailing launches: workgroups per CU (0: one per tile)
+    int t2_per_cu = 0;                   // FP64 second-stream trailing launches: workgroups per CU (0: one per tile)
     int64_t small_max = 0;               // FP64: a level's small supernodes go to one k_small_level launch
                                          // when it has at most this many of them (0: never)
     int64_t nsmall = 0;                  // supernodes the plan factors that way
@@ -653,6 +653,7 @@ static int flatten_upload(mxc_factor *F) {
         const bool by_panel = !F->deterministic && !F->fold_trsm;
         auto paneled = [&](int64_t s) { return by_panel && F->Super[s + 1] - F->Super[s] > 16; };
         constexpr size_t PSTEPS = PANEL / NB;
+        const std::vector<UpdDesc> *pending_t2 = nullptr;    // forked, launched after the next panel
         auto edge_of = [&](const UpdDesc &u) { return F->tune[kind_of(L_TRAIL)][tile_bucket(u.M, u.N, u.K)]; };
         for (size_t t = 0; t < nst; t++) {
             const StepBlocks &sb = F->blk_steps[l][t];
@@ -695,6 +696,13 @@ static int flatten_upload(mxc_factor *F) {
                     }
                 if ((long long)panels.size() > b)
                     F->factor_launches.push_back(Launch{L_PANEL, b, (long long)panels.size() - b, 0});
+                // the previous panel's second-stream update after this panel's launch:
+                // the panel's workgroups get their CUs first, and in a replayed graph the
+                // first branch recorded continues on its predecessor's queue
+                if (pending_t2) {
+                    emit(L_TRAIL2, *pending_t2, true);
+                    pending_t2 = nullptr;
+                }
             }
             // blocks of at most TINY_DIAG columns: one lane each; at most 16: one
             // wave each; wider blocks: a workgroup each
@@ -830,12 +838,14 @@ static int flatten_upload(mxc_factor *F) {
             }
             if (fork_t2) {
                 // the second-stream update starts when this step's own trailing
-                // update has finished, together with the next diagonal block's
-                // factorization: that single workgroup then finds a CU before the
-                // second stream's tiles fill them all (started beside the trailing
-                // update, it waited for the whole second-stream launch to drain)
+                // update has finished, behind the next panel's launch (started
+                // before it, uncapped, it filled the CUs and the panel waited for it
+                // to drain; capped at three workgroups per CU it lost 15% of its
+                // rate: 80^3 27-point FP64 factor 48.7 ms capped, 46.5 ms uncapped
+                // behind the panel)
                 F->factor_launches.push_back(Launch{L_FORK, 0, 0, 0});
-                emit(L_TRAIL2, sb.trail2, true);
+                if (by_panel) pending_t2 = &sb.trail2;
+                else emit(L_TRAIL2, sb.trail2, true);
                 level_forked = true;
             }
             fused_s.clear();
@@ -1716,10 +1726,8 @@ template <typename T, int MODE, bool PD = false>
 static void launch_tile(mxc_factor *F, const Launch &L, T *W, hipStream_t st = nullptr) {
     if (!st) st = F->stream;
     if constexpr (std::is_same<T, double>::value && MODE == MODE_TRAIL && !PD) {
-        // FP64 second-stream update: a grid of t2_per_cu workgroups per CU that
-        // walk all its tiles, so that every CU keeps room for a diagonal
-        // factorization of the main stream (k_potrf_diag: 144 registers per
-        // lane and 66.5 KB of LDS beside three 96-register, 17 KB tiles)
+        // FP64 second-stream update, when capped: a grid of t2_per_cu workgroups
+        // per CU that walk all its tiles
         const long long cap = ((long long)F->t2_per_cu * device_cus()) / 8 * 8;
         if (L.kind == L_TRAIL2 && L.tile == 64 && cap > 0 && L.count > cap) {
             hipLaunchKernelGGL((k_tile_grid<double, MODE_TRAIL, 64>), dim3((unsigned)cap), dim3(256), 0, st,
