@@ -318,6 +318,7 @@ struct mxc_factor {
     // tile edge per (M, N) bucket: 32 up to 64 x 32, 128 for M > 128 and N > 32,
     // else 64 (mxc_set_tile overrides an entry before the plan is built)
     int tune[NKIND][NBUCKET];
+    bool tiles_default = true;             // no table set or tuned by the caller
 
     // hipGraph replay: the launch sequence depends only on the pattern, so it is
     // captured once and replayed for every refactorization / solve
@@ -508,9 +509,24 @@ static int flatten_upload(mxc_factor *F) {
         long long n16 = 0;
         for (const UpdDesc &u : blocks) n16 += tiny16(u) ? 1 : 0;
         const bool use16 = n16 >= 200000;
+        // FP32 descendant updates of more than 128 rows and 64 columns take 128-wide
+        // split-FP16 tiles (half the operand bytes per product) where they make at least
+        // two workgroups per CU; a level with fewer leaves CUs idle with them (41^3 FP32
+        // factor 2.27 ms with 64-wide tiles throughout, 2.37 ms with 128; 80^3 27-point
+        // 26.9 and 25.2 ms).  FP64 tiles of 128 were slower in both.  A table that the
+        // caller set or tuned is taken as it is.
+        auto wide128 = [&](const UpdDesc &u) {
+            return F->precision != MXC_FP64 && F->split16 && F->tiles_default && kind == L_UPD && u.M > 128 &&
+                   u.N > 64 && u.K > 32;
+        };
+        long long n128 = 0;
+        if (F->precision != MXC_FP64 && F->tiles_default && kind == L_UPD)
+            for (const UpdDesc &u : blocks) n128 += wide128(u) ? lower_tiles(u, 128, lower_only) : 0;
+        const bool use128 = n128 >= 2 * 256;
         auto edge = [&](size_t bi) {
             const UpdDesc &u = blocks[bi];
             if (force && (*force)[bi] > 0) return (*force)[bi];
+            if (use128 && wide128(u)) return 128;
             return (use16 && tiny16(u)) ? 16 : F->tune[kind_of(kind)][tile_bucket(u.M, u.N, u.K)];
         };
         long long total = 0;
@@ -2791,6 +2807,7 @@ static int autotune_impl(mxc_factor *F, int reps, int *table) {
             F->tune[kind][b] = best_ts;
         }
     }
+    F->tiles_default = false;
     F->values_loaded = false;        // the timing launches scribbled on L
     int rc = flatten_upload(F);
     if (rc) return rc;
@@ -2814,6 +2831,7 @@ extern "C" int mxc_set_tiles(mxc_factor *F, const int *table) {
         if (table[q] != 32 && table[q] != 64 && table[q] != 128) return MXC_INVALID;
     for (int k = 0; k < NKIND; k++)
         for (int b = 0; b < NBUCKET; b++) F->tune[k][b] = table[k * NBUCKET + b];
+    F->tiles_default = false;
     return flatten_upload(F);
 }
 
