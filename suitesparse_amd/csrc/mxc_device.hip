@@ -3170,10 +3170,10 @@ static int updown_run(mxc_factor *F, int update, int64_t ncol, const int64_t *Cp
                                (const long long *)(dm + oi), (const double *)(dm + ov), (long long)sidx.size(), Wc);
         for (const UdLaunch &L : launches) {
             if (L.nb > 0)
-                hipLaunchKernelGGL(k_updown_block<T>, dim3((unsigned)L.nb), dim3(64), 0, sm, d_blocks + L.b0, W, Wc,
+                hipLaunchKernelGGL(k_updown_block<T>, dim3((unsigned)L.nb), dim3(UD_THREADS), 0, sm, d_blocks + L.b0, W, Wc,
                                    alpha, par, update, dbound, F->d_mflag);
             if (L.nr > 0)
-                hipLaunchKernelGGL(k_updown_rows<T>, dim3((unsigned)L.nr), dim3(64), 0, sm, d_blocks,
+                hipLaunchKernelGGL(k_updown_rows<T>, dim3((unsigned)L.nr), dim3(UD_THREADS), 0, sm, d_blocks,
                                    d_rows + L.r0, W, (const int *)F->d_Ls, Wc, (const T *)par);
         }
         HIPTRY(hipGetLastError());
