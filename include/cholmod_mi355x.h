@@ -332,11 +332,11 @@ int mxc_solve_refine(mxc_factor *F, const double *B, int64_t nrhs, double *X, in
  * same factor; off by default because the waiting tiles hold their CUs
  * through the diagonal factorization, which costs more than the launch. */
 #define MXC_OPT_FOLD_TRSM 7
-/* MXC_OPT_T2_GRID (default 0, FP64 factors): the look-ahead's second-stream
+/* MXC_OPT_T2_GRID (default 3, FP64 factors): the look-ahead's second-stream
  * trailing update runs on a grid of this many workgroups per CU, each walking
- * its share of the tiles (0: one workgroup per tile).  With a cap every CU
- * keeps room for the main stream's launches; the next panel's launch is
- * recorded before the update and takes its CUs first, so no cap is fastest. */
+ * its share of the tiles (0: one workgroup per tile).  Every CU then keeps
+ * room for the main stream's diagonal factorizations, which otherwise wait
+ * for the whole second-stream launch to drain. */
 #define MXC_OPT_T2_GRID 8
 /* MXC_OPT_SMALL_FUSED (default 0, FP64 factors): in every etree level with at
  * most this many supernodes of at most 16 columns and 64 rows that have

@@ -230,7 +230,7 @@ class Factor:
 
     def set_t2_grid(self, per_cu: int):
         """FP64: workgroups per CU of the look-ahead's second-stream trailing update,
-        each walking its share of the tiles (default 0: one workgroup per tile)."""
+        each walking its share of the tiles (default 3; 0: one workgroup per tile)."""
         check("mxc_set_option", lib().mxc_set_option(self._num, 8, int(per_cu)))
 
     def set_small_fused(self, max_per_level):

@@ -1076,303 +1076,6 @@ __global__ __launch_bounds__(256) void k_potrf_diag(const DiagTask *__restrict__
     potrf_block<T, SAFE>(tasks[blockIdx.x], W, SX, SX + NB * PS, sfail, fail, adiag, rho, rd, tmp);
 }
 
-
-// ---------------------------------------------------------------------------
-// Panel factorization: the 64-column steps of a panel (up to 384 columns) of
-// every supernode of a level that has one, in one launch.  A workgroup owns
-// 64 rows of a panel and walks the panel's column blocks s = 0, 1, ...
-// (left-looking):
-//   C = sum_{b < s} L[r, b] L[s, b]'          rows r: its own, MFMA, K = 64 s
-//   L[r, s] = (A[r, s] - C) inv(L_ss)'        MFMA, with the published inverse
-// The workgroup of diagonal block t adds L[t, s] L[t, s]' to the sum for its
-// own block as each L[t, s] is formed, so that once L[t, t-1] is known only
-// one 64-wide product and the block's factorization (potrf_core) are left;
-// it publishes its rows (for the C of rows below) before, and the inverse
-// after that.
-//
-// What bounds it: the chain of diagonal blocks (hand-off, inverse load, TRSM,
-// product, potrf_core: 17 us per 64 columns, of which potrf_core 8); the
-// launches per step that this replaces (TRSM, then trailing tiles with the next
-// block's factorization as a tail) took 50 us per step at 64^3.  64 rows per
-// workgroup: a panel of the largest supernodes (14,600 rows) is then 229
-// workgroups, one per CU, and small ones still spread.
-//
-// Hand-off: as in the chained sweeps (kernels_solve.h), published blocks and
-// flags are stored and loaded by device-scope atomics, performed at the device
-// coherence point; a publisher waits for its stores (s_waitcnt) before the
-// barrier that precedes the flag store, and a consumer issues its loads after
-// its flag load returned.  All other data are a workgroup's own.  Tasks are
-// ordered by diagonal block, then the rows below, and a workgroup waits only
-// for diagonal blocks before its own: for workgroups of lower index, which
-// have started.  A wait is bounded (FOLD_SPIN polls); past that it raises
-// *abort and the host reports a device error.
-// ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ T dev_load(const T *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-template <typename T>
-__device__ __forceinline__ void dev_store(T *p, T v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// Wave-uniform wait until *flag != 0 or the wait gives up.
-__device__ __forceinline__ void panel_wait(const int *flag, int *abort) {
-    for (int it = 1; __builtin_amdgcn_readfirstlane(dev_load(flag)) == 0; it++) {
-        __builtin_amdgcn_s_sleep(1);
-        if ((it & 63) == 0 && (it >= FOLD_SPIN || __builtin_amdgcn_readfirstlane(dev_load(abort)) != 0)) {
-            dev_store(abort, 1);
-            break;
-        }
-    }
-    asm volatile("" ::: "memory");          // the published data's loads stay after the flag load
-}
-
-// Every thread's published stores are done, then the flag.
-__device__ __forceinline__ void panel_publish(int *flag) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    if (threadIdx.x == 0) dev_store(flag, 1);
-}
-
-// Row stride of the panel workgroups' two 64 x 64 buffers: two workgroups of
-// doubles fit a CU's 160 KB.
-constexpr int PANEL_LD = NB + 4;
-
-template <typename T, bool SAFE, bool DIAG>
-__device__ __forceinline__ void panel_rows(const PanelTask &t, T *__restrict__ W, const int *__restrict__ Ls,
-                                           unsigned *__restrict__ Lh, const double *__restrict__ adiag,
-                                           int *__restrict__ fail, double rho, const Redo &rd,
-                                           int *__restrict__ ready, int *__restrict__ abort, T *smem) {
-    typedef typename MfmaOp<T>::acc_t acc_t;
-    constexpr int LD = PANEL_LD;
-    T(*Am)[LD] = reinterpret_cast<T(*)[LD]>(smem);              // Am[j][i]: the block of A, then of L
-    T(*Im)[LD] = reinterpret_cast<T(*)[LD]>(smem + NB * LD);    // Im[k][j] = inv(j, k)
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);     // (a scalar: offsets by w need no vector registers)
-    const int l15 = lane & 15, l4 = lane >> 4;
-    const int nsteps = DIAG ? t.blk : (t.ncols + NB - 1) / NB;
-    T *Wr = W + t.lx + t.r0;                                    // the workgroup's rows, column 0
-    auto own = [](const T *p) { return DIAG ? dev_load(p) : *p; };
-    int ex = 0;                                                 // FP32: the split-FP16 scale of row 16 w + l15
-    const bool h16 = std::is_same<T, float>::value && Lh;
-    if (h16 && 16 * w + l15 < t.nr) ex = row_scale_exp(adiag, Ls[t.ls + t.r0 + 16 * w + l15]);
-
-    // the diagonal block: lower 16x16 blocks q = w, w + 4, w + 8 of the column-by-column list
-    constexpr int NDB = DIAG ? 3 : 1;
-    const int dbi[3] = {w, w == 3 ? 2 : w + 1, 3}, dbj[3] = {0, w == 3 ? 2 : 1, w == 0 ? 2 : 3};
-    const int nd = w < 2 ? 3 : 2;
-    acc_t accD[NDB];
-#pragma unroll
-    for (int q = 0; q < NDB; q++) accD[q] = acc_t{0, 0, 0, 0};
-    // its sum over one more block of the workgroup's rows, held in Am
-    auto product = [&]() {
-#pragma unroll
-        for (int q = 0; q < NDB; q++)
-            if (q < nd) {
-#pragma unroll
-                for (int kk = 0; kk < NB; kk += 4)
-                    accD[q] = MfmaOp<T>::mma(Am[kk + l4][16 * dbj[q] + l15], Am[kk + l4][16 * dbi[q] + l15], accD[q]);
-            }
-    };
-
-    for (int s = 0; s < nsteps; s++) {
-        const int nbs = min(NB, t.ncols - s * NB);
-        T *Ws = Wr + (long long)s * NB * t.ld;                  // the block's column 0
-        if (DIAG && s > 0) {
-            product();
-            // the last block's device-scope stores are complete (every thread's,
-            // with the barrier) before the loads of the workgroup's own rows below:
-            // a device-scope load may pass a store of another wave in flight
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();                                    // and Am is staged into below
-        }
-        // C on 2 x 2 waves of 2 x 2 MFMA blocks
-        const int wr = w & 1, wc = w >> 1;
-        acc_t acc[2][2];
-#pragma unroll
-        for (int m = 0; m < 2; m++)
-#pragma unroll
-            for (int n = 0; n < 2; n++) acc[m][n] = acc_t{0, 0, 0, 0};
-        constexpr int CK = 32, PER = CK / 4;
-        T g[16];                                                // loads in flight: X and Y of a stage, or A
-        auto fetch_a = [&]() {
-#pragma unroll
-            for (int e = 0; e < 16; e++)
-                g[e] = Ws[min(32 * wr + 16 * ((e >> 2) & 1) + l15, t.nr - 1) +
-                          (long long)min(32 * wc + 16 * (e >> 3) + MfmaOp<T>::row(lane, e & 3), nbs - 1) * t.ld];
-        };
-        if (s == 0) fetch_a();
-        if (s > 0) {
-            panel_wait(ready + t.flag + 2 * s, abort);
-            // 32 columns per stage (in Am and Im, free until the sums are complete):
-            // its 32 products per wave cover the latency of the next stage's loads
-            const T *xrow = W + t.lx + s * NB, *yrow = Wr;
-            const int xr = min(lane, nbs - 1), yr = min(lane, t.nr - 1);
-            auto fetch = [&](int k0) {
-#pragma unroll
-                for (int q = 0; q < PER; q++) {
-                    const long long o = (long long)(k0 + w + 4 * q) * t.ld;
-                    g[q] = dev_load(xrow + o + xr);
-                    g[PER + q] = own(yrow + o + yr);
-                }
-            };
-            fetch(0);
-            for (int k0 = 0; k0 < s * NB; k0 += CK) {
-                if (k0 > 0) __syncthreads();                    // the previous stage's reads are done
-#pragma unroll
-                for (int q = 0; q < PER; q++) {
-                    Im[w + 4 * q][lane] = g[q];
-                    Am[w + 4 * q][lane] = g[PER + q];
-                }
-                __syncthreads();
-                if (k0 + CK < s * NB) fetch(k0 + CK);
-                else fetch_a();
-#pragma unroll
-                for (int kk = 0; kk < CK; kk += 4) {
-                    T xa[2], yb[2];
-#pragma unroll
-                    for (int m = 0; m < 2; m++) xa[m] = Im[kk + l4][32 * wc + 16 * m + l15];
-#pragma unroll
-                    for (int n = 0; n < 2; n++) yb[n] = Am[kk + l4][32 * wr + 16 * n + l15];
-#pragma unroll
-                    for (int m = 0; m < 2; m++)
-#pragma unroll
-                        for (int n = 0; n < 2; n++) acc[m][n] = MfmaOp<T>::mma(xa[m], yb[n], acc[m][n]);
-                }
-            }
-            __syncthreads();                                    // the staged columns' reads are done
-        }
-#pragma unroll
-        for (int m = 0; m < 2; m++)
-#pragma unroll
-            for (int n = 0; n < 2; n++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    const int j = 32 * wc + 16 * m + MfmaOp<T>::row(lane, v);
-                    Am[j][32 * wr + 16 * n + l15] = j < nbs ? g[8 * m + 4 * n + v] - acc[m][n][v] : (T)0;
-                }
-        // the inverse of block s
-        panel_wait(ready + t.flag + 2 * s + 1, abort);
-        const T *inv = W + t.winv + (long long)s * NB * NB;
-        T iv[16];
-#pragma unroll
-        for (int q = 0; q < 16; q++) iv[q] = dev_load(inv + min(lane, nbs - 1) + min(w + 4 * q, nbs - 1) * nbs);
-#pragma unroll
-        for (int q = 0; q < 16; q++) Im[w + 4 * q][lane] = (lane < nbs && w + 4 * q < nbs) ? iv[q] : (T)0;
-        __syncthreads();
-        // L(i, j) = sum_{k <= j} A(i, k) inv(j, k): wave w forms rows 16 w .. 16 w + 15
-        acc_t l[4];
-#pragma unroll
-        for (int jb = 0; jb < 4; jb++) l[jb] = acc_t{0, 0, 0, 0};
-#pragma unroll
-        for (int kk = 0; kk < NB; kk += 4) {
-            const T b = Am[kk + l4][16 * w + l15];
-#pragma unroll
-            for (int jb = kk / 16; jb < 4; jb++)
-                l[jb] = MfmaOp<T>::mma(Im[kk + l4][16 * jb + l15], b, l[jb]);
-        }
-        const int i = 16 * w + l15;
-#pragma unroll
-        for (int jb = 0; jb < 4; jb++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int j = 16 * jb + MfmaOp<T>::row(lane, v);
-                if (i < t.nr && j < nbs) {
-                    T *p = Ws + i + (long long)j * t.ld;
-                    if constexpr (DIAG) dev_store(p, l[jb][v]);
-                    else *p = l[jb][v];
-                    if (h16) Lh[p - W] = split_pack((float)l[jb][v], ex);
-                }
-            }
-        if constexpr (DIAG) {
-            // (rows 16 w .. of Am are read by wave w alone above)
-#pragma unroll
-            for (int jb = 0; jb < 4; jb++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) Am[16 * jb + MfmaOp<T>::row(lane, v)][i] = l[jb][v];
-        }
-        __syncthreads();                                        // Am is complete, Im free
-    }
-
-    if constexpr (DIAG) {
-        __shared__ int sfail[2];
-        T *S = smem, *X = smem + NB * PS;
-        T *Wd = Wr + (long long)t.r0 * t.ld;
-        const int nb = t.nr;
-        T dv[3][4];
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-#pragma unroll
-            for (int v = 0; v < 4; v++)
-                dv[q][v] = Wd[min(16 * dbi[q] + l15, nb - 1) +
-                              (long long)min(16 * dbj[q] + MfmaOp<T>::row(lane, v), nb - 1) * t.ld];
-        if (nsteps > 0) {
-            product();
-            __syncthreads();                                    // Am's reads are done (S takes its place)
-        }
-#pragma unroll
-        for (int q = 0; q < 3; q++) {
-            if (q >= nd) break;
-            const int i = 16 * dbi[q] + l15;
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int j = 16 * dbj[q] + MfmaOp<T>::row(lane, v);
-                const bool in = i < nb && j < nb;
-                const T a = dv[q][v] - accD[q][v];
-                S[i * PS + j] = in ? a : (i == j ? (T)1 : (T)0);
-                // the FP64 redo starts from the updated block in W
-                if (SAFE && in && j <= i) Wd[i + (long long)j * t.ld] = a;
-            }
-        }
-        potrf_init(X, sfail);
-        // (the rows' stores have had the product's time to complete)
-        panel_publish(ready + t.flag + 2 * t.blk);
-        const int col0 = t.col0 + t.blk * NB;
-        potrf_core<T, SAFE>(S, X, sfail, nb, adiag, col0, rho);
-        int *flag = ready + t.flag + 2 * t.blk + 1;
-        const long long winv = t.winv + (long long)t.blk * NB * NB;
-        if (SAFE && sfail[1]) {
-            __shared__ double tmp[NB];
-            const DiagTask dt{t.lx + t.r0 + (long long)t.r0 * t.ld, winv, t.ld, nb, col0, 0};
-            redo_block64<T>(dt, W, reinterpret_cast<double *>(smem), tmp, sfail, tid, 256, rd, fail,
-                            [] { __syncthreads(); });
-            __threadfence();
-            panel_publish(flag);
-            return;
-        }
-        const int i = tid & (NB - 1), c0 = tid >> 6;
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const int c = c0 + 4 * q;
-            if (i < nb && c < nb) dev_store(W + winv + i + (long long)c * nb, c <= i ? X[i * PS + c] : (T)0);
-        }
-        panel_publish(flag);
-        if (tid == 0 && sfail[0] >= 0) atomicMin(fail, col0 + sfail[0]);
-#pragma unroll
-        for (int q = 0; q < 16; q++) {
-            const int c = c0 + 4 * q;
-            if (i < nb && c <= i) Wd[i + (long long)c * t.ld] = S[i * PS + c];
-        }
-    }
-}
-
-template <typename T, bool SAFE>
-__global__ __launch_bounds__(256, 2) void k_panel(const PanelTask *__restrict__ tasks, T *__restrict__ W,
-                                                  const int *__restrict__ Ls, unsigned *__restrict__ Lh,
-                                                  const double *__restrict__ adiag, int *__restrict__ fail,
-                                                  double rho, Redo rd, int *__restrict__ ready,
-                                                  int *__restrict__ abort) {
-    __shared__ __attribute__((aligned(16))) T smem[2 * NB * PANEL_LD];
-    static_assert(PS <= PANEL_LD, "the diagonal block and its inverse fit the staging buffers");
-    const PanelTask t = tasks[blockIdx.x];
-    // the chain of diagonal blocks goes ahead of the second stream's trailing
-    // tiles on its CUs (wave priority: 80^3 27-point FP64 54.0 -> 53.6 ms)
-    if (t.blk >= 0) __builtin_amdgcn_s_setprio(3);
-    if (t.blk >= 0) panel_rows<T, SAFE, true>(t, W, Ls, Lh, adiag, fail, rho, rd, ready, abort, smem);
-    else panel_rows<T, SAFE, false>(t, W, Ls, Lh, adiag, fail, rho, rd, ready, abort, smem);
-}
-
 // Diagonal blocks of at most 16 columns (the many tiny supernodes of the
 // lower etree levels): one wave per block, four blocks per workgroup, the
 // block and its inverse from one elimination (panel_elim).
@@ -1567,8 +1270,7 @@ __global__ __launch_bounds__(256) void k_trsm_tiny(const UpdDesc *__restrict__ d
 // panel_elim's pivot arithmetic (r_j = 1/sqrt(d_jj), L_jj = d_jj r_j,
 // L_rj = a_rj r_j, a non-positive pivot reported and replaced by 1) applied
 // to the rows below the diagonal block as well, which makes the TRSM part of
-// the same pass.  The inverse of the diagonal block is formed as potrf16_wave
-// forms it, column c by lane c.
+// the same pass.  Column c of the diagonal block's inverse is formed by lane c.
 // ---------------------------------------------------------------------------
 constexpr int SMALL_COLS = 16;
 constexpr int SMALL_NROW = 64;

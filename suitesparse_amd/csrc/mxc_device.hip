@@ -153,12 +153,11 @@ static inline int kind_of(int launch_kind) {
 // L_BQUAD: its quarter-wave supernodes, sixteen lanes each; L_DIAG_TINY:
 // diagonal blocks of at most TINY_DIAG columns, one lane each; L_TRSM_TINY:
 // the panel TRSM of tiny supernodes, one lane each; L_SMALL: a level's small
-// supernodes (FP64), each factored whole by one wave (k_small_level); L_PANEL:
-// the 64-column steps of one panel of a level's supernodes (k_panel).
+// supernodes (FP64), each factored whole by one wave (k_small_level).
 enum { L_UPD = 0, L_DIAG = 1, L_TRSM = 2, L_TRAIL = 3, L_FSTEP = 4, L_BSTEP = 5, L_FSMALL = 6, L_BSMALL = 7,
        L_DIAG_SMALL = 8, L_TRAIL2 = 9, L_FORK = 10, L_JOIN = 11, L_FCHAIN = 12, L_BCHAIN = 13,
        L_TRAILD = 14, L_FTINY = 15, L_BTINY = 16, L_DIAG_TINY = 17, L_TRSM_TINY = 18, L_FQUAD = 19,
-       L_BQUAD = 20, L_SMALL = 21, L_PANEL = 22 };
+       L_BQUAD = 20, L_SMALL = 21 };
 
 // ---------------------------------------------------------------------------
 // device memory pool: one hipMalloc, sub-allocated first-fit with coalescing
@@ -239,13 +238,10 @@ struct mxc_factor {
     bool chain = true;                   // solves: one chained launch per level
     bool diag_tails = true;              // trailing launches factor the next diagonal blocks
     bool fold_trsm = false;              // FP64: ... and apply the next step's TRSM (UpdDesc::fold)
-    int *d_ready = nullptr;              // per diagonal task: published by a folding tail; then the
-                                         // panel factorizations' flags; last, the abort flag
-    int64_t nready = 0;                  // entries of d_ready
-    int64_t panel_flags = 0;             // first of the panel factorizations' flags in d_ready
-    PanelTask *d_panel = nullptr;
+    int *d_ready = nullptr;              // per diagonal task: published by a folding tail; + abort flag
+    int64_t nready = 0;                  // diagonal tasks covered by d_ready
     bool merge_t2 = true;                // FP64: fold second-stream updates into later trailing launches
-    int t2_per_cu = 0;                   // FP64 second-stream trailing launches: workgroups per CU (0: one per tile)
+    int t2_per_cu = 3;                   // FP64 second-stream trailing launches: workgroups per CU (0: one per tile)
     int64_t small_max = 0;               // FP64: a level's small supernodes go to one k_small_level launch
                                          // when it has at most this many of them (0: never)
     int64_t nsmall = 0;                  // supernodes the plan factors that way
@@ -462,8 +458,6 @@ static int flatten_upload(mxc_factor *F) {
     std::vector<Tile> tiles;
     std::vector<DiagTask> diags;
     std::vector<SmallTask> smalls;
-    std::vector<PanelTask> panels;
-    long long npflag = 0;                // panel flags handed out
     F->factor_launches.clear();
     int64_t nupd = 0;
     // FP64: supernodes of at most SMALL_COLS columns and SMALL_NROW rows that
@@ -662,64 +656,9 @@ static int flatten_upload(mxc_factor *F) {
         // column slices and their supernodes
         std::vector<std::vector<UpdDesc>> merged(nst);
         std::vector<std::vector<int64_t>> merged_s(nst);
-        // Supernodes wider than 16 columns take their 64-column steps a panel at a time
-        // (k_panel), except where an option is about the separate launches of a step:
-        // the deterministic mode keeps the summation order of its right-looking steps,
-        // and a folded TRSM belongs to a trailing launch.
-        const bool by_panel = !F->deterministic && !F->fold_trsm;
-        auto paneled = [&](int64_t s) { return by_panel && F->Super[s + 1] - F->Super[s] > 16; };
-        constexpr size_t PSTEPS = PANEL / NB;
-        const std::vector<UpdDesc> *pending_t2 = nullptr;    // forked, launched after the next panel
         auto edge_of = [&](const UpdDesc &u) { return F->tune[kind_of(L_TRAIL)][tile_bucket(u.M, u.N, u.K)]; };
         for (size_t t = 0; t < nst; t++) {
             const StepBlocks &sb = F->blk_steps[l][t];
-            if (by_panel && t % PSTEPS == 0) {
-                const long long b = (long long)panels.size();
-                std::vector<PanelTask> heads;
-                for (size_t q = 0; q < sb.diags.size(); q++) {
-                    const int64_t s = sb.diag_s[q];
-                    if (!paneled(s)) continue;
-                    const int64_t nscol = F->Super[s + 1] - F->Super[s], nsrow = F->Lpi[s + 1] - F->Lpi[s];
-                    const int64_t c0 = (int64_t)t * NB;
-                    PanelTask x{};
-                    x.lx = sb.diags[q].off;
-                    x.winv = sb.diags[q].winv;
-                    x.ld = (int)nsrow;
-                    x.ncols = (int)std::min<int64_t>(PANEL, nscol - c0);
-                    x.col0 = sb.diags[q].col0;
-                    x.ls = (int)(F->Lpi[s] + c0);
-                    x.flag = (int)npflag;
-                    x.nr = (int)(nsrow - c0);            // rows of the panel, for the loop below
-                    npflag += 2 * ceil_div(x.ncols, NB);
-                    heads.push_back(x);
-                }
-                for (int k = 0; k < (int)PSTEPS; k++)    // diagonal blocks in chain order
-                    for (const PanelTask &h : heads) {
-                        if (k * NB >= h.ncols) continue;
-                        PanelTask x = h;
-                        x.r0 = k * NB;
-                        x.nr = std::min(NB, h.ncols - k * NB);
-                        x.blk = k;
-                        panels.push_back(x);
-                    }
-                for (const PanelTask &h : heads)         // then the rows below
-                    for (int r = h.ncols; r < h.nr; r += NB) {
-                        PanelTask x = h;
-                        x.r0 = r;
-                        x.nr = std::min(NB, h.nr - r);
-                        x.blk = -1;
-                        panels.push_back(x);
-                    }
-                if ((long long)panels.size() > b)
-                    F->factor_launches.push_back(Launch{L_PANEL, b, (long long)panels.size() - b, 0});
-                // the previous panel's second-stream update after this panel's launch:
-                // the panel's workgroups get their CUs first, and in a replayed graph the
-                // first branch recorded continues on its predecessor's queue
-                if (pending_t2) {
-                    emit(L_TRAIL2, *pending_t2, true);
-                    pending_t2 = nullptr;
-                }
-            }
             // blocks of at most TINY_DIAG columns: one lane each; at most 16: one
             // wave each; wider blocks: a workgroup each
             for (int cls = 2; cls >= 0; cls--) {
@@ -727,7 +666,7 @@ static int flatten_upload(mxc_factor *F) {
                 for (size_t q = 0; q < sb.diags.size(); q++) {
                     const DiagTask &d = sb.diags[q];
                     if (std::binary_search(fused_s.begin(), fused_s.end(), sb.diag_s[q])) continue;
-                    if (fused_here(t, sb.diag_s[q]) || paneled(sb.diag_s[q])) continue;
+                    if (fused_here(t, sb.diag_s[q])) continue;
                     const int c = d.nb <= TINY_DIAG ? 2 : d.nb <= 16 ? 1 : 0;
                     if (c == cls) diags.push_back(d);
                 }
@@ -743,7 +682,7 @@ static int flatten_upload(mxc_factor *F) {
                 for (size_t q = 0; q < sb.trsm.size(); q++) {
                     const UpdDesc &u = sb.trsm[q];
                     if (std::binary_search(folded_s.begin(), folded_s.end(), sb.trsm_s[q])) continue;
-                    if (fused_here(t, sb.trsm_s[q]) || paneled(sb.trsm_s[q])) continue;
+                    if (fused_here(t, sb.trsm_s[q])) continue;
                     if (u.K <= TINY_DIAG && u.M <= TINY_TRSM_ROWS) {
                         descs.push_back(u);
                         descs.back().pd = -1;
@@ -771,7 +710,7 @@ static int flatten_upload(mxc_factor *F) {
                 // their diagonal tails (under graph replay the second stream's branch
                 // ran after the main one).  Each slice takes its supernode's own
                 // trailing edge; every merged launch must stay within the tail limit.
-                bool merge = F->merge_t2 && F->precision == MXC_FP64 && t + 3 < nst && !by_panel;
+                bool merge = F->merge_t2 && F->precision == MXC_FP64 && t + 3 < nst;
                 std::vector<std::vector<UpdDesc>> add(3);
                 std::vector<std::vector<int64_t>> add_s(3);
                 for (size_t q = 0; merge && q < sb.trail2.size(); q++) {
@@ -832,11 +771,7 @@ static int flatten_upload(mxc_factor *F) {
                                   sb.trail[q].N >= NB && sb.trail[q].M == nx.trsm[rt].M + NB;
                 }
             }
-            if (by_panel) {
-                // (a supernode with a trailing block has more than 64 columns) only the
-                // update of the next panel's columns, at a panel's last step
-                if (t % PSTEPS == PSTEPS - 1) emit(L_TRAIL, sb.trail, true);
-            } else if (merged[t].empty()) {
+            if (merged[t].empty()) {
                 emit(L_TRAIL, sb.trail, true, &follow, &fused, nullptr, &foldable, &folded);
             } else {
                 // this step's trailing blocks, then the merged slices at their
@@ -854,14 +789,12 @@ static int flatten_upload(mxc_factor *F) {
             }
             if (fork_t2) {
                 // the second-stream update starts when this step's own trailing
-                // update has finished, behind the next panel's launch (started
-                // before it, uncapped, it filled the CUs and the panel waited for it
-                // to drain; capped at three workgroups per CU it lost 15% of its
-                // rate: 80^3 27-point FP64 factor 48.7 ms capped, 46.5 ms uncapped
-                // behind the panel)
+                // update has finished, together with the next diagonal block's
+                // factorization: that single workgroup then finds a CU before the
+                // second stream's tiles fill them all (started beside the trailing
+                // update, it waited for the whole second-stream launch to drain)
                 F->factor_launches.push_back(Launch{L_FORK, 0, 0, 0});
-                if (by_panel) pending_t2 = &sb.trail2;
-                else emit(L_TRAIL2, sb.trail2, true);
+                emit(L_TRAIL2, sb.trail2, true);
                 level_forked = true;
             }
             fused_s.clear();
@@ -882,8 +815,6 @@ static int flatten_upload(mxc_factor *F) {
     ffree(F, F->d_tiles);
     ffree(F, F->d_diag);
     ffree(F, F->d_small);
-    ffree(F, F->d_panel);
-    F->d_panel = nullptr;
     F->d_desc = nullptr;
     F->d_tiles = nullptr;
     F->d_diag = nullptr;
@@ -895,15 +826,12 @@ static int flatten_upload(mxc_factor *F) {
     if ((rc = dupload(F, &F->d_tiles, tiles, F->stream))) return rc;
     if ((rc = dupload(F, &F->d_diag, diags, F->stream))) return rc;
     if (!smalls.empty() && (rc = dupload(F, &F->d_small, smalls, F->stream))) return rc;
-    if (!panels.empty() && (rc = dupload(F, &F->d_panel, panels, F->stream))) return rc;
-    // publication flags of the diagonal tasks (folded TRSMs) and of the panel
-    // factorizations + the wait-abort flag
+    // publication flags of the diagonal tasks (folded TRSMs) + the wait-abort flag
     ffree(F, F->d_ready);
     F->d_ready = nullptr;
     F->nready = 0;
-    F->panel_flags = (int64_t)diags.size();
-    F->nready = F->panel_flags + npflag + 1;
-    if ((rc = dalloc(F, &F->d_ready, (size_t)F->nready))) return rc;
+    if ((rc = dalloc(F, &F->d_ready, diags.size() + 1))) return rc;
+    F->nready = (int64_t)diags.size() + 1;
     if (F->precision != MXC_FP64) {
         // FP32 factors: room in the FP64 redo queue for every diagonal task
         ffree(F, F->d_redo);
@@ -1469,7 +1397,7 @@ extern "C" void mxc_factor_free(mxc_factor *F) {
                     F->d_diag, F->d_stask, F->d_fail, F->d_adiag, F->d_rowptr, F->d_src, F->d_col,
                     F->d_vals, F->d_Ax, F->d_norm, F->d_beta, F->d_work, F->d_part, F->d_b, F->d_x, F->d_r,
                     F->d_cnt, F->d_abort, F->d_seg, F->d_segout, F->d_pinv, F->d_redo, F->d_ready,
-                    F->d_mw, F->d_mpar, F->d_malpha, F->d_mflag, F->d_mdesc, F->d_small, F->d_panel};
+                    F->d_mw, F->d_mpar, F->d_malpha, F->d_mflag, F->d_mdesc, F->d_small};
     for (void *p : ptrs) ffree(F, p);
 
     for (hipEvent_t e : F->ev) (void)hipEventDestroy(e);
@@ -1604,7 +1532,7 @@ extern "C" int mxc_factor_stats(const mxc_factor *F, int64_t *counts, double *ms
                 case L_UPD: counts[0]++; break;
                 case L_DIAG: case L_DIAG_SMALL: case L_DIAG_TINY: case L_SMALL: counts[1]++; break;
                 case L_TRSM: case L_TRSM_TINY: counts[2]++; break;
-                case L_TRAIL: case L_TRAIL2: case L_TRAILD: case L_PANEL: counts[3]++; break;
+                case L_TRAIL: case L_TRAIL2: case L_TRAILD: counts[3]++; break;
                 default: break;
             }
         }
@@ -1742,8 +1670,9 @@ template <typename T, int MODE, bool PD = false>
 static void launch_tile(mxc_factor *F, const Launch &L, T *W, hipStream_t st = nullptr) {
     if (!st) st = F->stream;
     if constexpr (std::is_same<T, double>::value && MODE == MODE_TRAIL && !PD) {
-        // FP64 second-stream update, when capped: a grid of t2_per_cu workgroups
-        // per CU that walk all its tiles
+        // FP64 second-stream update: a grid of t2_per_cu workgroups per CU that
+        // walk all its tiles, so that every CU keeps room for a diagonal
+        // factorization of the main stream
         const long long cap = ((long long)F->t2_per_cu * device_cus()) / 8 * 8;
         if (L.kind == L_TRAIL2 && L.tile == 64 && cap > 0 && L.count > cap) {
             hipLaunchKernelGGL((k_tile_grid<double, MODE_TRAIL, 64>), dim3((unsigned)cap), dim3(256), 0, st,
@@ -1909,19 +1838,6 @@ static int enqueue_factor(mxc_factor *F) {
                 launch_tile<T, MODE_TRAIL, true>(F, L, W);
                 F->counts[3]++;
                 break;
-            case L_PANEL: {
-                const dim3 g((unsigned)L.count), b(256);
-                int *flags = F->d_ready + F->panel_flags, *ab = F->d_ready + (F->nready - 1);
-                unsigned *Lh = std::is_same<T, float>::value && F->split16 ? F->d_Lh : nullptr;
-                if (safe)
-                    hipLaunchKernelGGL((k_panel<T, true>), g, b, 0, sm, F->d_panel + L.begin, W, F->d_Ls, Lh,
-                                       (const double *)F->d_adiag, F->d_fail, F->rho, rq, flags, ab);
-                else
-                    hipLaunchKernelGGL((k_panel<T, false>), g, b, 0, sm, F->d_panel + L.begin, W, F->d_Ls, Lh,
-                                       (const double *)F->d_adiag, F->d_fail, 0.0, rq, flags, ab);
-                F->counts[3]++;
-                break;
-            }
             case L_TRAIL2:
                 launch_tile<T, MODE_TRAIL>(F, L, W, two ? F->stream2 : sm);
                 F->counts[3]++;
@@ -2006,7 +1922,7 @@ extern "C" int mxc_factorize(mxc_factor *F, const double *Ax, int location, doub
         HIPTRY(hipMemcpyAsync(&wait_abort, F->d_ready + (F->nready - 1), sizeof(int), hipMemcpyDeviceToHost, sm));
     HIPTRY(hipStreamSynchronize(sm));
     if (wait_abort) {
-        snprintf(g_err, sizeof(g_err), "factorization: a wait for a diagonal block did not end");
+        snprintf(g_err, sizeof(g_err), "factorization: a folded TRSM gave up waiting for its diagonal block");
         return MXC_GPU_PROBLEM;
     }
     {

@@ -57,20 +57,6 @@ struct DiagTask {
     int pad;
 };
 
-// One workgroup of a panel factorization (k_panel): 64 rows (at most) of a
-// panel of up to 384 columns of a supernode.
-struct PanelTask {
-    long long lx;      // W offset of the panel's first diagonal element
-    long long winv;    // W offset of the inverse of its block 0 (64 x 64 blocks follow)
-    int ld;            // nsrow of the supernode
-    int ncols;         // columns of the panel
-    int r0, nr;        // the workgroup's rows, counted from the panel's first row
-    int blk;           // its diagonal block, or -1 for rows below the panel's columns
-    int col0;          // global column of the panel's first column
-    int ls;            // Ls position of the panel's first row
-    int flag;          // ready[flag + 2t]: rows of block t published, [flag + 2t + 1]: its inverse
-};
-
 // A small supernode factored whole by one wave (k_small_level): its
 // descendant updates are descs[u0 .. u0 + nu), in descendant order.
 struct SmallTask {
