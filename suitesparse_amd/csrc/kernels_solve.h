@@ -777,7 +777,12 @@ __global__ __launch_bounds__(256) void k_sweep_small_bwd(const SweepTask *__rest
 // LDS once per pass.
 // ---------------------------------------------------------------------------
 constexpr int CHAIN_SPIN = 1 << 22;
-constexpr int CHAIN_RHS = 4;   // columns per launch (the host splits wider right-hand sides)
+// Columns per launch (the host splits wider right-hand sides): the chain of
+// blocks and the reads of L are paid per launch, so eight columns cost little
+// more than four, where two launches of four cost twice (64^3 diffusion FP64,
+// 8 columns: 3.99 ms as 4 + 4, 3.15 ms as 8; 41^3 FP32 factor + refinement, 5
+// columns: 5.91 ms as 4 + 1, 5.30 ms as 8).
+constexpr int CHAIN_RHS = 8;
 
 template <typename T>
 __device__ __forceinline__ T ld_dev(const T *p) {
@@ -830,13 +835,18 @@ __device__ __forceinline__ T lane_get(T v, int l) {
     }
 }
 
-// acc[z] += sum_j l[j] q(j + 16 z), q(m) = lane m's value of q (wave-uniform)
-template <typename T, int ZC>
-__device__ __forceinline__ void fma_bcast(T (&acc)[ZC], const T (&l)[16], T q) {
+// acc[z] += sum_j l[j] q[z / 4](j + 16 (z % 4)), q(m) = lane m's value of q (wave-uniform)
+template <typename T, int ZC, int NQ>
+__device__ __forceinline__ void fma_bcast(T (&acc)[ZC], const T (&l)[16], const T (&q)[NQ]) {
+    // four columns at a time (all the broadcasts at once spill scalar registers)
 #pragma unroll
-    for (int z = 0; z < ZC; z++)
+    for (int j0 = 0; j0 < 16; j0 += 4) {
 #pragma unroll
-        for (int j = 0; j < 16; j++) acc[z] += l[j] * lane_get(q, j + 16 * z);
+        for (int z = 0; z < ZC; z++)
+#pragma unroll
+            for (int j = j0; j < j0 + 4; j++) acc[z] += l[j] * lane_get(q[z / 4], j + 16 * (z % 4));
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
 // Forward.  Task fields: c0 / nb = block t (diag workgroup, pad[0] = 0) or
@@ -853,7 +863,8 @@ __global__ __launch_bounds__(256) void k_chain_fwd(const SweepTask *__restrict__
     __shared__ T red[4][ZC][NB];
     __shared__ T vs[ZC][NB];
     const SweepTask t = tasks[blockIdx.x];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // (a scalar: its offsets too)
     const bool below = t.pad[0] != 0;
     const int row = (below ? t.r0 : t.c0) + lane;  // the lane's row of the supernode
     const bool rok = row < (below ? t.r1 : t.c0 + t.nb);
@@ -872,7 +883,8 @@ __global__ __launch_bounds__(256) void k_chain_fwd(const SweepTask *__restrict__
         for (int j = 0; j < 16; j++)
             l[j] = (rok && c + j < t.nscol) ? Lr[(long long)(b * NB + j) * t.nsrow] : (T)0;
     };
-    const int qz = lane >> 4, qj = lane & 15;      // the value lane q loads: column qj, rhs qz
+    const int qz = lane >> 4, qj = lane & 15;      // the values lane q loads: column qj, rhs qz and qz + 4
+    constexpr int NQ = (ZC + 3) / 4;
     int seen = 0;
     for (int z0 = 0; z0 < nrhs; z0 += ZC) {
         const int zc = min(ZC, nrhs - z0);
@@ -885,8 +897,13 @@ __global__ __launch_bounds__(256) void k_chain_fwd(const SweepTask *__restrict__
             if (b + 1 < nblk) load_blk(ln, b + 1);
             if (seen <= b) seen = chain_wait(mycnt, b + 1, abort);
             const int c = b * NB + 16 * w + qj;
-            const T q = (qz < zc && c < t.nscol) ? ld_dev(X + t.k1 + c + (long long)(z0 + qz) * n) : (T)0;
-            fma_bcast<T, ZC>(acc, lc, q);
+            T q[NQ];
+#pragma unroll
+            for (int e = 0; e < NQ; e++) {
+                const T v = ld_dev(X + t.k1 + min(c, t.nscol - 1) + (long long)(z0 + min(qz + 4 * e, zc - 1)) * n);
+                q[e] = (qz + 4 * e < zc && c < t.nscol) ? v : (T)0;
+            }
+            fma_bcast<T, ZC, NQ>(acc, lc, q);
 #pragma unroll
             for (int j = 0; j < 16; j++) lc[j] = ln[j];
         }
@@ -948,7 +965,8 @@ __global__ __launch_bounds__(256) void k_chain_bwd(const SweepTask *__restrict__
     __shared__ T vs[ZC][NB];
     __shared__ T tile[4][16][NB + 1];              // per wave: 16 rows x 64 columns of L
     const SweepTask t = tasks[blockIdx.x];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const bool below = t.pad[0] != 0;
     const int nblk = t.np, tb = t.c0 / NB;
     const int col = t.c0 + lane;                   // the lane's column of the supernode
@@ -992,7 +1010,8 @@ __global__ __launch_bounds__(256) void k_chain_bwd(const SweepTask *__restrict__
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     };
-    const int qz = lane >> 4, qj = lane & 15;      // the value lane q loads: row qj, rhs qz
+    const int qz = lane >> 4, qj = lane & 15;      // the values lane q loads: row qj, rhs qz and qz + 4
+    constexpr int NQ = (ZC + 3) / 4;
     int seen = 0;
     bool slots_ready = false;
     for (int z0 = 0; z0 < nrhs; z0 += ZC) {
@@ -1009,8 +1028,14 @@ __global__ __launch_bounds__(256) void k_chain_bwd(const SweepTask *__restrict__
                 get(lc);
                 if (r + NB < t.r1) fetch(gn, r + NB, t.r1);
                 const int rq = r + 16 * w + qj;
-                const T q = (qz < zc && rq < t.r1) ? X[Ls[t.psi + rq] + (long long)(z0 + qz) * n] : (T)0;
-                fma_bcast<T, ZC>(acc, lc, q);
+                const long long gq = Ls[t.psi + min(rq, t.r1 - 1)];
+                T q[NQ];
+#pragma unroll
+                for (int e = 0; e < NQ; e++) {
+                    const T v = X[gq + (long long)(z0 + min(qz + 4 * e, zc - 1)) * n];
+                    q[e] = (qz + 4 * e < zc && rq < t.r1) ? v : (T)0;
+                }
+                fma_bcast<T, ZC, NQ>(acc, lc, q);
                 if (r + NB < t.r1) put(gn);
             }
 #pragma unroll
@@ -1043,8 +1068,13 @@ __global__ __launch_bounds__(256) void k_chain_bwd(const SweepTask *__restrict__
             if (b - 1 > tb) fetch(gn, (b - 1) * NB, t.nscol);
             if (seen < nblk - b) seen = chain_wait(cnt + t.p0, nblk - b, abort);
             const int rq = b * NB + 16 * w + qj;
-            const T q = (qz < zc && rq < t.nscol) ? ld_dev(X + t.k1 + rq + (long long)(z0 + qz) * n) : (T)0;
-            fma_bcast<T, ZC>(acc, lc, q);
+            T q[NQ];
+#pragma unroll
+            for (int e = 0; e < NQ; e++) {
+                const T v = ld_dev(X + t.k1 + min(rq, t.nscol - 1) + (long long)(z0 + min(qz + 4 * e, zc - 1)) * n);
+                q[e] = (qz + 4 * e < zc && rq < t.nscol) ? v : (T)0;
+            }
+            fma_bcast<T, ZC, NQ>(acc, lc, q);
             if (b - 1 > tb) put(gn);
         }
 #pragma unroll

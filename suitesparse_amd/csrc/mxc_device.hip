@@ -2078,8 +2078,10 @@ static void launch_chain(mxc_factor *F, const Launch &L, T *Xw, int nr, T *part)
             hipLaunchKernelGGL((k_chain_fwd<T, 1>), g, b, 0, sm, tk, W, F->d_Ls, Xw, n, nr, F->d_cnt, F->d_abort);
         else if (nr == 2)
             hipLaunchKernelGGL((k_chain_fwd<T, 2>), g, b, 0, sm, tk, W, F->d_Ls, Xw, n, nr, F->d_cnt, F->d_abort);
-        else
+        else if (nr <= 4)
             hipLaunchKernelGGL((k_chain_fwd<T, 4>), g, b, 0, sm, tk, W, F->d_Ls, Xw, n, nr, F->d_cnt, F->d_abort);
+        else
+            hipLaunchKernelGGL((k_chain_fwd<T, 8>), g, b, 0, sm, tk, W, F->d_Ls, Xw, n, nr, F->d_cnt, F->d_abort);
     } else {
         if (nr == 1)
             hipLaunchKernelGGL((k_chain_bwd<T, 1>), g, b, 0, sm, tk, W, F->d_Ls, Xw, part, n, nr,
@@ -2087,8 +2089,11 @@ static void launch_chain(mxc_factor *F, const Launch &L, T *Xw, int nr, T *part)
         else if (nr == 2)
             hipLaunchKernelGGL((k_chain_bwd<T, 2>), g, b, 0, sm, tk, W, F->d_Ls, Xw, part, n, nr,
                                F->d_cnt, F->d_abort);
-        else
+        else if (nr <= 4)
             hipLaunchKernelGGL((k_chain_bwd<T, 4>), g, b, 0, sm, tk, W, F->d_Ls, Xw, part, n, nr,
+                               F->d_cnt, F->d_abort);
+        else
+            hipLaunchKernelGGL((k_chain_bwd<T, 8>), g, b, 0, sm, tk, W, F->d_Ls, Xw, part, n, nr,
                                F->d_cnt, F->d_abort);
     }
 }
