@@ -267,7 +267,7 @@ __device__ __forceinline__ void redo_block64(const DiagTask &t, T *__restrict__ 
     }
 }
 
-template <typename T, bool SAFE>
+template <typename T, bool SAFE, bool LOADED = false>
 __device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W, T *S, T *X, int *sfail,
                                             int *__restrict__ fail, const double *__restrict__ adiag,
                                             double rho, const Redo &rd, double *tmp);
@@ -297,7 +297,9 @@ struct PdArgs {
 constexpr int FOLD_SPIN = 1 << 22;
 
 // The tail itself: S and X of potrf_block carved from the tile's LDS buffer.
-template <typename T>
+// LOADED: the tile's epilogue has put the block into S (tail_entry); else it is
+// read back from W.
+template <typename T, bool LOADED>
 __device__ __forceinline__ void pd_tail(const PdArgs &pda, int pd, T *__restrict__ W, unsigned char *smem,
                                         const double *__restrict__ adiag, bool publish) {
     __shared__ int sfail[2];
@@ -305,14 +307,21 @@ __device__ __forceinline__ void pd_tail(const PdArgs &pda, int pd, T *__restrict
     T *S = reinterpret_cast<T *>(smem);
     if (pda.rho > 0) {
         __shared__ double tmp[NB];
-        potrf_block<T, true>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, tmp);
+        potrf_block<T, true, LOADED>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, tmp);
     } else {
-        potrf_block<T, false>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, nullptr);
+        potrf_block<T, false, LOADED>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, nullptr);
     }
     if (publish) {
         __syncthreads();                    // every wave's stores of L and the inverse are issued
         if (threadIdx.x == 0) __hip_atomic_store(pda.ready + pd, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// Entry (i, j) of the block that a tail factors (nb columns, extended by the
+// identity), a its value in the trailing tile.
+template <typename T>
+__device__ __forceinline__ T tail_entry(int i, int j, int nb, T a) {
+    return i < nb && j < nb ? (j <= i ? a : (T)0) : (i == j ? (T)1 : (T)0);
 }
 
 // Wait (whole workgroup) until *flag != 0 or the wait gives up.
@@ -372,6 +381,8 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     const int i0 = tl.ti * TS, j0 = tl.tj * TS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wr = TS <= 32 ? 0 : (wave & 1), wc = TS <= 32 ? 0 : (wave >> 1);
+    const bool tail = PD && d.pd >= 0 && tl.ti == 0 && tl.tj == 0;   // factors the next diagonal block
+    if (tail) __builtin_amdgcn_s_setprio(3);    // on the critical path: ahead of the CU's other tiles
 
     // thread t stages row r = t % TS of chunk rows k = t/TS + KG*q, q < PER.  The
     // loads are unconditional (rows and k clamped into the block, a predicated
@@ -440,6 +451,25 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
 #pragma unroll
         for (int b = 0; b < MB; b++) acc[a][b] = acc_t{0, 0, 0, 0};
 
+    // trailing tiles: the entries of C, loaded together and unconditionally, clamped
+    // into the block (a predicated read-modify-write each waited for its own round
+    // trip).  A launch with tails waits for its diagonal tile, so there the loads go
+    // under the last chunk's products; elsewhere, and in tiles of 128, a row of MFMA
+    // blocks at a time in the epilogue, which leaves the registers for another
+    // resident tile (80^3 27-point FP64 pass 56.1 ms, 58.4 ms with all ahead).  FP32
+    // factor 28.9 -> 27.4 ms at 80^3 27-point, 2.95 -> 2.74 ms at 41^3; FP64
+    // 15.06 -> 14.94 ms at 64^3.
+    constexpr int OM = MODE != MODE_TRAIL ? 0 : PD && MB <= 2 ? MB : 1;
+    T old[OM > 0 ? OM : 1][MB][4];
+    auto load_c = [&](int m, int o) {
+#pragma unroll
+        for (int n = 0; n < MB; n++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                old[o][n][v] = W[d.c_off + (long long)min(j0 + wc * WB + m * 16 + MfmaOp<T>::row(lane, v), d.N - 1) * d.ldc +
+                                 min(i0 + wr * WB + n * 16 + (lane & 15), d.M - 1)];
+    };
+
     int buf = 0;
     for (int k0 = 0; k0 < d.K; k0 += BK) {
         if (NBUF == 1 && k0 > 0) __syncthreads();   // the previous chunk's reads are done
@@ -449,7 +479,12 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
             Xs[buf][kq + KG * q][r] = rx[q];
         }
         __syncthreads();
-        if (k0 + BK < d.K) fetch(k0 + BK);      // next chunk in flight during the MFMAs
+        if (k0 + BK < d.K) {
+            fetch(k0 + BK);                     // next chunk in flight during the MFMAs
+        } else if constexpr (OM > 1) {
+#pragma unroll
+            for (int m = 0; m < OM; m++) load_c(m, m);
+        }
         // operands one step ahead: their LDS latency passes under the MFMAs
         // (with the unconditional loads, one 64-wide FP64 launch over 6000 x 5600,
         // K = 384: 55.5 -> 60.5 TFLOP/s; a chunk alone on its CU 2,190 -> 1,920
@@ -478,7 +513,11 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     const bool fold = CAN_FOLD && d.fold && d.pd >= 0 && tl.tj == 0 && tl.ti >= 1;
     T (*Af)[TS + LDS_PAD] = reinterpret_cast<T (*)[TS + LDS_PAD]>(smem);               // Af[k][i]
     T (*If)[TS + LDS_PAD] = reinterpret_cast<T (*)[TS + LDS_PAD]>(smem + FOLD_HALF);   // If[k][j]
-    if (CAN_FOLD && fold) __syncthreads();     // every wave is done with the staged chunks
+    // the tail's block goes to LDS as well as to W
+    constexpr bool TAIL_LDS = PD && TS == NB;
+    T *S = reinterpret_cast<T *>(smem);
+    const int tail_nb = TAIL_LDS && tail ? pda.diags[d.pd].nb : 0;
+    if ((CAN_FOLD && fold) || (TAIL_LDS && tail)) __syncthreads();   // every wave is done with the staged chunks
 
     // FP32 TRSM with Lh: the panel is also stored in split-FP16 form, each row
     // scaled by its own exponent, for the update and trailing tiles that read it
@@ -497,6 +536,7 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     //                                   j = j0 + WB*wc + 16m + row(lane, v)
 #pragma unroll
     for (int m = 0; m < MB; m++) {
+        if constexpr (OM == 1) load_c(m, 0);
 #pragma unroll
         for (int n = 0; n < MB; n++) {
             const int il = wr * WB + n * 16 + (lane & 15);
@@ -505,16 +545,17 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
             for (int v = 0; v < 4; v++) {
                 const int jl = wc * WB + m * 16 + MfmaOp<T>::row(lane, v);
                 const int j = j0 + jl;
-                if (i >= d.M || j >= d.N) continue;
                 const T c = acc[m][n][v];
+                if (TAIL_LDS && tail) S[il * PS + jl] = tail_entry(il, jl, tail_nb, old[OM > 1 ? m : 0][n][v] - c);
+                if (i >= d.M || j >= d.N) continue;
                 if (MODE == MODE_SCATTER) {
                     if (i < j) continue;
                     atomic_sub(W + d.c_off + (long long)relc[jl] * d.ldc + relr[il], c);
                 } else if (MODE == MODE_TRAIL) {
                     if (i < j) continue;
-                    T *w = W + d.c_off + (long long)j * d.ldc + i;
-                    if (CAN_FOLD && fold) Af[jl][il] = *w - c;   // the next TRSM's input, kept here
-                    else *w -= c;
+                    const T a = old[OM > 1 ? m : 0][n][v] - c;
+                    if (CAN_FOLD && fold) Af[jl][il] = a;        // the next TRSM's input, kept here
+                    else W[d.c_off + (long long)j * d.ldc + i] = a;
                 } else {
                     W[d.c_off + (long long)j * d.ldc + i] = c;
                     if (std::is_same<T, float>::value && Lh)
@@ -563,7 +604,7 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
         }
     }
     if constexpr (PD) {
-        if (d.pd >= 0 && tl.ti == 0 && tl.tj == 0) pd_tail<T>(pda, d.pd, W, smem, adiag, d.fold != 0);
+        if (tail) pd_tail<T, TAIL_LDS>(pda, d.pd, W, smem, adiag, d.fold != 0);
     }
 }
 
@@ -644,6 +685,8 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
     const int i0 = tl.ti * TS, j0 = tl.tj * TS;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wr = wave & 1, wc = wave >> 1;
+    const bool tail = PD && d.pd >= 0 && tl.ti == 0 && tl.tj == 0;   // as in tile_work
+    if (tail) __builtin_amdgcn_s_setprio(3);
 
     for (int e = tid; e < 2 * TS; e += NT) {
         if (e < TS) {
@@ -729,13 +772,30 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
 #pragma unroll
         for (int b = 0; b < MB; b++) acc[a][b] = f32x4{0, 0, 0, 0};
 
+    // the entries of C, as in tile_work
+    constexpr int OM = MODE != MODE_TRAIL ? 0 : PD && MB <= 2 ? MB : 1;
+    float old[OM > 0 ? OM : 1][MB][4];
+    auto load_c = [&](int m, int o) {
+#pragma unroll
+        for (int n = 0; n < MB; n++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                old[o][n][v] = W[d.c_off + (long long)min(j0 + wc * WB + m * 16 + 4 * (lane >> 4) + v, d.N - 1) * d.ldc +
+                                 min(i0 + wr * WB + n * 16 + (lane & 15), d.M - 1)];
+    };
+
     fetch(0);
     const int ko = 8 * (lane >> 4);
     for (int k0 = 0; k0 < d.K; k0 += BKH) {
         __syncthreads();                         // the previous chunk's reads are done
         stage(k0);
         __syncthreads();
-        if (k0 + BKH < d.K) fetch(k0 + BKH);     // next chunk in flight during the MFMAs
+        if (k0 + BKH < d.K) {
+            fetch(k0 + BKH);                     // next chunk in flight during the MFMAs
+        } else if constexpr (OM > 1) {
+#pragma unroll
+            for (int m = 0; m < OM; m++) load_c(m, m);
+        }
         half8_t xh[MB], xl[MB], yh[MB], yl[MB];
 #pragma unroll
         for (int m = 0; m < MB; m++) {
@@ -761,8 +821,13 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
 
     // epilogue: acc[m][n][v] = C(i, j) 2^(s_i + s_j), i = i0 + WB*wr + 16n + lane%16,
     //                                               j = j0 + WB*wc + 16m + 4 (lane/16) + v
+    constexpr bool TAIL_LDS = PD && TS == NB;
+    float *S = reinterpret_cast<float *>(smem);
+    const int tail_nb = TAIL_LDS && tail ? pda.diags[d.pd].nb : 0;
+    if (TAIL_LDS && tail) __syncthreads();       // every wave is done with the staged chunks
 #pragma unroll
     for (int m = 0; m < MB; m++) {
+        if constexpr (OM == 1) load_c(m, 0);
 #pragma unroll
         for (int n = 0; n < MB; n++) {
             const int il = wr * WB + n * 16 + (lane & 15);
@@ -771,17 +836,18 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
             for (int v = 0; v < 4; v++) {
                 const int jl = wc * WB + m * 16 + 4 * (lane >> 4) + v;
                 const int j = j0 + jl;
-                if (i >= d.M || j >= d.N || i < j) continue;
                 const float c = ldexpf(acc[m][n][v], -(exr[il] + exc[jl]));
+                if (TAIL_LDS && tail) S[il * PS + jl] = tail_entry(il, jl, tail_nb, old[OM > 1 ? m : 0][n][v] - c);
+                if (i >= d.M || j >= d.N || i < j) continue;
                 if (MODE == MODE_SCATTER)
                     atomic_sub(W + d.c_off + (long long)relc[jl] * d.ldc + relr[il], c);
                 else
-                    W[d.c_off + (long long)j * d.ldc + i] -= c;
+                    W[d.c_off + (long long)j * d.ldc + i] = old[OM > 1 ? m : 0][n][v] - c;
             }
         }
     }
     if constexpr (PD) {
-        if (d.pd >= 0 && tl.ti == 0 && tl.tj == 0) pd_tail<float>(pda, d.pd, W, smem, adiag, false);
+        if (tail) pd_tail<float, TAIL_LDS>(pda, d.pd, W, smem, adiag, false);
     }
 }
 
@@ -1022,14 +1088,14 @@ __device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const
 // sfail: two shared ints, the first failing column and the breakdown flag;
 // tmp: NB shared doubles for the redo) and writes L_tt and the inverse back
 // to W.
-template <typename T, bool SAFE>
+template <typename T, bool SAFE, bool LOADED>
 __device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W, T *S, T *X, int *sfail,
                                             int *__restrict__ fail, const double *__restrict__ adiag,
                                             double rho, const Redo &rd, double *tmp) {
     const int tid = threadIdx.x;
     const int nb = t.nb;
     const int i = tid & (NB - 1), c0 = tid >> 6;
-    {
+    if constexpr (!LOADED) {
         // all 16 loads of a thread in flight at once (unconditional, from inside the
         // block: a predicated load is a branch each), then the LDS stores
         T v[16];
