@@ -267,8 +267,30 @@ __device__ __forceinline__ void redo_block64(const DiagTask &t, T *__restrict__ 
     }
 }
 
+// Where potrf_core keeps block (i, j), i >= j, of the inverse, in elements from
+// its block S.  FP64: off-diagonal blocks take the place of S's unused blocks
+// (j, i), diagonal ones stand side by side in 16 rows below S: 42 KB, so that
+// three workgroups of a trailing kernel with tails share a CU instead of two
+// (64^3 diffusion factor 14.99 -> 14.75 ms, 80^3 27-point 52.7 -> 52.0 ms).
+// FP32, whose FP64 redo needs the 33 KB anyway: a square of its own below S
+// (its addresses are cheaper: 41^3 factor 2.75 ms, 2.80 ms in FP64's places).
+template <typename T>
+__device__ __forceinline__ int inv_at(int i, int j) {
+    if (std::is_same<T, float>::value) return (NB + 16 * i) * PS + 16 * j;
+    return i == j ? NB * PS + 16 * i : 16 * j * PS + 16 * i;
+}
+
+// LDS of potrf_block, in bytes: the block and its inverse, and with `redo` at
+// least the FP64 redo's block.
+template <typename T>
+constexpr size_t potrf_lds(bool redo) {
+    const size_t own = sizeof(T) * (std::is_same<T, float>::value ? 2 * NB : NB + 16) * PS;
+    const size_t r64 = redo ? sizeof(double) * NB * (NB + 1) : 0;
+    return own > r64 ? own : r64;
+}
+
 template <typename T, bool SAFE, bool LOADED = false>
-__device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W, T *S, T *X, int *sfail,
+__device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W, T *S, int *sfail,
                                             int *__restrict__ fail, const double *__restrict__ adiag,
                                             double rho, const Redo &rd, double *tmp);
 
@@ -296,7 +318,7 @@ struct PdArgs {
 
 constexpr int FOLD_SPIN = 1 << 22;
 
-// The tail itself: S and X of potrf_block carved from the tile's LDS buffer.
+// The tail itself: potrf_block in the tile's LDS buffer.
 // LOADED: the tile's epilogue has put the block into S (tail_entry); else it is
 // read back from W.
 template <typename T, bool LOADED>
@@ -307,9 +329,9 @@ __device__ __forceinline__ void pd_tail(const PdArgs &pda, int pd, T *__restrict
     T *S = reinterpret_cast<T *>(smem);
     if (pda.rho > 0) {
         __shared__ double tmp[NB];
-        potrf_block<T, true, LOADED>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, tmp);
+        potrf_block<T, true, LOADED>(pda.diags[pd], W, S, sfail, pda.fail, adiag, pda.rho, pda.rd, tmp);
     } else {
-        potrf_block<T, false, LOADED>(pda.diags[pd], W, S, S + NB * PS, sfail, pda.fail, adiag, pda.rho, pda.rd, nullptr);
+        potrf_block<T, false, LOADED>(pda.diags[pd], W, S, sfail, pda.fail, adiag, pda.rho, pda.rd, nullptr);
     }
     if (publish) {
         __syncthreads();                    // every wave's stores of L and the inverse are issued
@@ -342,7 +364,7 @@ __device__ __forceinline__ void fold_wait(const int *flag, int *abort) {
 
 // One tile of a launch: virtual workgroup bx of g (k_tile: the workgroup
 // itself; k_tile_grid: each of its workgroups takes bx, bx + grid, ...).
-template <typename T, int MODE, int TS, bool PD>
+template <typename T, int MODE, int TS, bool PD, bool FOLD>
 __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, const Tile *__restrict__ tiles,
                                           T *__restrict__ W, const int *__restrict__ Ls, unsigned *__restrict__ Lh,
                                           const double *__restrict__ adiag, const PdArgs &pda, const int bx,
@@ -361,10 +383,13 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     // waves per SIMD either way and keeps two buffers.
     constexpr int NBUF = TS == 128 ? 2 : 1;
     constexpr size_t XY_BYTES = sizeof(T) * NBUF * BK * (TS + LDS_PAD);
-    constexpr size_t PD_BYTES = PD ? sizeof(T) * 2 * NB * PS : 0;
+    constexpr size_t PD_BYTES = PD ? potrf_lds<T>(std::is_same<T, float>::value) : 0;
     // folded TRSM (FP64, 64-wide trailing tiles): the updated block and the
     // next diagonal block's inverse, both k-major like the staged chunks
-    constexpr bool CAN_FOLD = PD && MODE == MODE_TRAIL && TS == NB && std::is_same<T, double>::value;
+    // (a variant of its own: its buffers, 69 KB, leave room for two workgroups per
+    // CU, the tail's 42 KB for three)
+    constexpr bool CAN_FOLD = FOLD;
+    static_assert(!FOLD || (PD && TS == NB && std::is_same<T, double>::value), "folded TRSM: FP64 tails");
     constexpr size_t FOLD_HALF = sizeof(T) * NB * (TS + LDS_PAD);
     constexpr size_t FOLD_BYTES = CAN_FOLD ? 2 * FOLD_HALF : 0;
     constexpr size_t SMEM0 = 2 * XY_BYTES > PD_BYTES ? 2 * XY_BYTES : PD_BYTES;
@@ -375,7 +400,7 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     __shared__ int relr[TS];
     __shared__ int relc[TS];
 
-    const int nf = PD ? pda.nfirst : 0;
+    const int nf = FOLD ? pda.nfirst : 0;
     const Tile tl = tiles[bx < nf ? bx : nf + xcd_tile(bx - nf, g - nf)];
     const UpdDesc d = descs[tl.desc];
     const int i0 = tl.ti * TS, j0 = tl.tj * TS;
@@ -608,7 +633,7 @@ __device__ __forceinline__ void tile_work(const UpdDesc *__restrict__ descs, con
     }
 }
 
-template <typename T, int MODE, int TS, bool PD = false>
+template <typename T, int MODE, int TS, bool PD = false, bool FOLD = false>
 __global__ __launch_bounds__(TS <= 32 ? 64 : 256, TS == 128 ? 2 : 1) void k_tile(const UpdDesc *__restrict__ descs,
                                                               const Tile *__restrict__ tiles,
                                                               T *__restrict__ W,
@@ -616,7 +641,7 @@ __global__ __launch_bounds__(TS <= 32 ? 64 : 256, TS == 128 ? 2 : 1) void k_tile
                                                               unsigned *__restrict__ Lh,
                                                               const double *__restrict__ adiag,
                                                               PdArgs pda = PdArgs{}) {
-    tile_work<T, MODE, TS, PD>(descs, tiles, W, Ls, Lh, adiag, pda, (int)blockIdx.x, (int)gridDim.x);
+    tile_work<T, MODE, TS, PD, FOLD>(descs, tiles, W, Ls, Lh, adiag, pda, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // The tiles of a launch on a grid of at most a few workgroups per CU (a
@@ -630,7 +655,7 @@ __global__ __launch_bounds__(256, 1) void k_tile_grid(const UpdDesc *__restrict_
                                                       int ntiles) {
     static_assert(TS >= 64, "four-wave tiles");
     for (int b = (int)blockIdx.x; b < ntiles; b += (int)gridDim.x) {
-        tile_work<T, MODE, TS, false>(descs, tiles, W, Ls, nullptr, adiag, PdArgs{}, b, ntiles);
+        tile_work<T, MODE, TS, false, false>(descs, tiles, W, Ls, nullptr, adiag, PdArgs{}, b, ntiles);
         __syncthreads();                   // the next tile restages the LDS buffers
     }
 }
@@ -671,7 +696,7 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
     static_assert(!PD || (MODE == MODE_TRAIL && TS >= 64), "diagonal tails: trailing tiles of 64 or 128");
     // one LDS buffer: the staged halves, reused by the diagonal-block tail
     constexpr size_t H_BYTES = 4 * sizeof(_Float16) * TS * RS;
-    constexpr size_t PD_BYTES = PD ? sizeof(float) * 2 * NB * PS : 0;
+    constexpr size_t PD_BYTES = PD ? potrf_lds<float>(true) : 0;
     __shared__ __attribute__((aligned(16))) unsigned char smem[H_BYTES > PD_BYTES ? H_BYTES : PD_BYTES];
     _Float16 *Xh = reinterpret_cast<_Float16 *>(smem);
     _Float16 *Xl = Xh + TS * RS;
@@ -980,19 +1005,19 @@ __device__ __forceinline__ int panel_elim(T (&a)[16], int nreal, T floor_l, bool
 
 // Factor and invert the diagonal block of nb columns held in LDS (256
 // threads).  S: the block, NB x PS row-major, its lower triangle (extended by
-// the identity past nb) on entry and L on return; X: its inverse, same layout,
-// the lower triangle's 16x16 blocks on return (blocks above the diagonal are
-// not written).  sfail[0] receives the first failing column (-1 on entry),
-// sfail[1] the breakdown flag (0 on entry).  X's four diagonal 16x16 blocks hold
-// the identity on entry (potrf_init).  The caller synchronizes before;
-// the block and its inverse are complete (and visible) on return.
+// the identity past nb) on entry and L on return.  Its inverse: the lower
+// triangle's 16x16 blocks at inv_at, in the same LDS.  sfail[0] receives the
+// first failing column (-1 on entry), sfail[1] the breakdown flag (0 on entry).
+// The inverse's four diagonal blocks hold the identity on entry (potrf_init).
+// The caller synchronizes before; the block and its inverse are complete (and
+// visible) on return.
 template <typename T>
-__device__ __forceinline__ void potrf_init(T *X, int *sfail) {
+__device__ __forceinline__ void potrf_init(T *S, int *sfail) {
     const int tid = threadIdx.x;
 #pragma unroll
     for (int q = 0; q < 4; q++) {
         const int e = tid + 256 * q, i = e >> 4, c = e & 15;
-        X[i * PS + (i & ~15) + c] = (i & 15) == c ? (T)1 : (T)0;
+        S[inv_at<T>(i >> 4, i >> 4) + (i & 15) * PS + c] = (i & 15) == c ? (T)1 : (T)0;
     }
     if (tid == 0) {
         sfail[0] = -1;
@@ -1001,7 +1026,7 @@ __device__ __forceinline__ void potrf_init(T *X, int *sfail) {
 }
 
 template <typename T, bool SAFE>
-__device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const double *__restrict__ adiag,
+__device__ __forceinline__ void potrf_core(T *S, int *sfail, int nb, const double *__restrict__ adiag,
                                            int col0, double rho) {
     typedef typename MfmaOp<T>::acc_t acc_t;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1014,12 +1039,12 @@ __device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const
 #pragma unroll
         for (int v = 0; v < 4; v++) S[(16 * i + (lane & 15)) * PS + 16 * j + MfmaOp<T>::row(lane, v)] -= acc[v];
     };
-    // X(p, j) = -X(p, p) T(p, j), T(p, j) held in X(p, j)
+    // X(p, j) = -X(p, p) T(p, j), T(p, j) held in the place of X(p, j)
     auto inv_row = [&](int p, int j) {
         acc_t acc = acc_t{0, 0, 0, 0};
-        mma_nn16<T>(X, 16 * p, 16 * p, X, 16 * p, 16 * j, acc, lane);
+        mma_nn16<T>(S + inv_at<T>(p, p), 0, 0, S + inv_at<T>(p, j), 0, 0, acc, lane);
         wave_sync_lds();                    // the wave's reads of T, before its stores
-        store16<T>(X, 16 * p, 16 * j, acc, lane, (T)-1, false);
+        store16<T>(S + inv_at<T>(p, j), 0, 0, acc, lane, (T)-1, false);
     };
     for (int p = 0; p < np; p++) {
         const int R = 16 * p;
@@ -1032,10 +1057,10 @@ __device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const
         }
         if (wave < 2) {
             // wave 0: row R + lane (past the last row: that row again, not stored);
-            // wave 1: the diagonal block's rows, then the identity rows X holds there
+            // wave 1: the diagonal block's rows, then the inverse's identity rows
             const bool row = R + lane < NB;
             const T *ar = (wave == 0 || lane < 16) ? S + min(R + lane, NB - 1) * PS + R
-                                                   : X + (R + (lane & 15)) * PS + R;
+                                                   : S + inv_at<T>(p, p) + (lane & 15) * PS;
             T a[16];
 #pragma unroll
             for (int c = 0; c < 16; c++) a[c] = ar[c];
@@ -1053,7 +1078,7 @@ __device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const
             } else if (lane >= 16 && lane < 32) {
                 // lane 16 + q: column q of the inverse
 #pragma unroll
-                for (int c = 0; c < 16; c++) X[(R + c) * PS + R + lane - 16] = a[c];
+                for (int c = 0; c < 16; c++) S[inv_at<T>(p, p) + c * PS + lane - 16] = a[c];
             }
         } else {
             // waves 2, 3: panel p-1's updates right of block column p, then T(p, j)
@@ -1064,8 +1089,8 @@ __device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const
             for (int j = 0; j < p; j++) {
                 if ((q++ & 1) != wave - 2) continue;
                 acc_t acc = acc_t{0, 0, 0, 0};
-                for (int k = j; k < p; k++) mma_nn16<T>(S, R, 16 * k, X, 16 * k, 16 * j, acc, lane);
-                store16<T>(X, R, 16 * j, acc, lane, (T)1, false);
+                for (int k = j; k < p; k++) mma_nn16<T>(S, R, 16 * k, S + inv_at<T>(k, j), 0, 0, acc, lane);
+                store16<T>(S + inv_at<T>(p, j), 0, 0, acc, lane, (T)1, false);
             }
         }
         __syncthreads();
@@ -1079,17 +1104,16 @@ __device__ __forceinline__ void potrf_core(T *S, T *X, int *sfail, int nb, const
 // SAFE (rho > 0, low-precision factor): a pivot d_jj <= rho * a_jj (a_jj the
 // assembled diagonal of A) signals breakdown of the block.  Its low-precision
 // result is dropped and the same workgroup refactors the block in FP64 in
-// place (redo_block64, in the LDS of S and X, which hold NB x (NB + 1)
-// doubles for T = float), before anything reads it.  Without SAFE a pivot
+// place (redo_block64, in the LDS of S and X), before anything reads it.  Without SAFE a pivot
 // <= 0 is reported as the failing column.
 //
 // potrf_block: the whole workgroup (256 threads) factors diagonal block t in
-// LDS (S: the block, X: its inverse, both NB x PS row-major and contiguous;
+// LDS (S: potrf_lds<T>(SAFE) bytes, potrf_core's layout;
 // sfail: two shared ints, the first failing column and the breakdown flag;
 // tmp: NB shared doubles for the redo) and writes L_tt and the inverse back
 // to W.
 template <typename T, bool SAFE, bool LOADED>
-__device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W, T *S, T *X, int *sfail,
+__device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W, T *S, int *sfail,
                                             int *__restrict__ fail, const double *__restrict__ adiag,
                                             double rho, const Redo &rd, double *tmp) {
     const int tid = threadIdx.x;
@@ -1110,13 +1134,11 @@ __device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W
             S[i * PS + c] = (i < nb && c < nb) ? (c <= i ? v[q] : (T)0) : (i == c ? (T)1 : (T)0);
         }
     }
-    potrf_init(X, sfail);
+    potrf_init(S, sfail);
     __syncthreads();
-    potrf_core<T, SAFE>(S, X, sfail, nb, adiag, t.col0, rho);
+    potrf_core<T, SAFE>(S, sfail, nb, adiag, t.col0, rho);
     if (SAFE && sfail[1]) {
         // breakdown: the block again from W, in FP64, in the LDS of S and X
-        static_assert(!SAFE || sizeof(T) * 2 * NB * PS >= sizeof(double) * NB * (NB + 1),
-                      "the FP64 redo needs the LDS of S and X");
         redo_block64<T>(t, W, reinterpret_cast<double *>(S), tmp, sfail, tid, 256, rd, fail,
                         [] { __syncthreads(); });
         return;
@@ -1127,7 +1149,10 @@ __device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W
         const int c = c0 + 4 * q;
         if (i < nb && c < nb) {
             if (c <= i) W[t.off + i + (long long)c * t.ld] = S[i * PS + c];
-            W[t.winv + i + (long long)c * nb] = (c <= i) ? X[i * PS + c] : (T)0;
+            W[t.winv + i + (long long)c * nb] =
+                c <= i ? S[std::is_same<T, float>::value ? (NB + i) * PS + c
+                                                         : inv_at<T>(i >> 4, c >> 4) + (i & 15) * PS + (c & 15)]
+                       : (T)0;
         }
     }
 }
@@ -1136,10 +1161,10 @@ template <typename T, bool SAFE>
 __global__ __launch_bounds__(256) void k_potrf_diag(const DiagTask *__restrict__ tasks,
                                                     T *__restrict__ W, int *__restrict__ fail,
                                                     const double *__restrict__ adiag, double rho, Redo rd) {
-    __shared__ __attribute__((aligned(16))) T SX[2 * NB * PS];   // the block and its inverse, row-major
+    __shared__ __attribute__((aligned(16))) T SX[potrf_lds<T>(SAFE) / sizeof(T)];   // the block and its inverse
     __shared__ int sfail[2];
     __shared__ double tmp[SAFE ? NB : 1];
-    potrf_block<T, SAFE>(tasks[blockIdx.x], W, SX, SX + NB * PS, sfail, fail, adiag, rho, rd, tmp);
+    potrf_block<T, SAFE>(tasks[blockIdx.x], W, SX, sfail, fail, adiag, rho, rd, tmp);
 }
 
 // Diagonal blocks of at most 16 columns (the many tiny supernodes of the

@@ -219,7 +219,6 @@ struct StepBlocks {
     std::vector<UpdDesc> trail2;   // right of the next panel (second stream)
     bool panel_end = false;        // trail holds the update of the next panel's columns
     std::vector<int64_t> diag_s, trail_s;   // supernode of each diag task / trail block
-    std::vector<int64_t> trail2_s;          // supernode of each trail2 block
     std::vector<int64_t> trsm_s;            // supernode of each TRSM block
 };
 
@@ -240,7 +239,6 @@ struct mxc_factor {
     bool fold_trsm = false;              // FP64: ... and apply the next step's TRSM (UpdDesc::fold)
     int *d_ready = nullptr;              // per diagonal task: published by a folding tail; + abort flag
     int64_t nready = 0;                  // diagonal tasks covered by d_ready
-    bool merge_t2 = true;                // FP64: fold second-stream updates into later trailing launches
     int t2_per_cu = 3;                   // FP64 second-stream trailing launches: workgroups per CU (0: one per tile)
     int64_t small_max = 0;               // FP64: a level's small supernodes go to one k_small_level launch
                                          // when it has at most this many of them (0: never)
@@ -428,29 +426,18 @@ static void drop_factor_graph(mxc_factor *F) {
 // Turn the host block lists into device descriptors, tiles and the launch
 // list, one launch per tile class (from F->tune) per phase.
 // FP64 trailing launches of at most this many tiles carry the next step's
-// diagonal blocks as tails: the FP64 tail kernels run at half the occupancy of
-// the plain ones (2 waves / SIMD, two resident workgroups per CU).  The FP32
-// tail kernels keep most of theirs and take tails in every trailing launch
-// (96^3 27-point FP32 factor: 72.3 ms unbounded, 73.0 ms at 512 tiles).
-constexpr long long PD_MAX_TILES_FP64 = 512;
+// diagonal blocks as tails: the FP64 tail kernels run at three resident
+// workgroups per CU, the plain ones at five.  64^3 diffusion FP64 pass 16.16 ms
+// at 512 tiles, 15.92 at 2048, 15.85 without a limit; 80^3 27-point 55.6, 55.0
+// and 55.3 ms.  The FP32 tail kernels keep most of their occupancy and take
+// tails in every trailing launch (96^3 27-point FP32 factor: 72.3 ms unbounded,
+// 73.0 ms at 512 tiles).
+constexpr long long PD_MAX_TILES_FP64 = 2048;
 
 // Tiles of edge ts over block u (its lower part when lower_only).
 static long long lower_tiles(const UpdDesc &u, int ts, bool lower_only) {
     const long long mt = ceil_div(u.M, ts), nt = ceil_div(u.N, ts);
     return lower_only ? mt * nt - nt * (nt - 1) / 2 : mt * nt;
-}
-
-// Columns [a, b) of trailing block u (relative to its first column): the
-// lower trapezoid of those columns, rows from a down.
-static UpdDesc column_slice(const UpdDesc &u, int a, int b) {
-    UpdDesc v = u;
-    v.x_off += a;
-    v.y_off += a;
-    v.c_off += a + (long long)a * u.ldc;
-    v.M = u.M - a;
-    v.N = b - a;
-    v.ls_off = u.ls_off + a;
-    return v;
 }
 
 static int flatten_upload(mxc_factor *F) {
@@ -483,14 +470,12 @@ static int flatten_upload(mxc_factor *F) {
     // follow[i] (trailing blocks): the next step's diagonal task of block i's
     // supernode, or null.  A block tiled at 64 or 128 gets it as its tail (pd);
     // fused[i] records that, so the next step's diagonal launch skips it.
-    // force[i] > 0 sets block i's tile edge (merged second-stream slices take the
-    // edge of their supernode's own trailing block, so they share its launch).
     // foldable[i] (trailing blocks, FP64): the next step's TRSM of block i's
     // supernode may be applied by block i's tiles (see UpdDesc::fold); folded[i]
     // records that it was (64-wide tiles with a tail), so that TRSM is skipped.
     auto emit = [&](int kind, const std::vector<UpdDesc> &blocks, bool lower_only,
                     const std::vector<const DiagTask *> *follow = nullptr, std::vector<char> *fused = nullptr,
-                    const std::vector<int> *force = nullptr, const std::vector<char> *foldable = nullptr,
+                    const std::vector<char> *foldable = nullptr,
                     std::vector<char> *folded = nullptr) {
         // FP64 descendant updates of at most 16 rows and columns take 16-wide tiles when a
         // level holds very many of them (the bottom levels of a forest of small systems:
@@ -519,7 +504,6 @@ static int flatten_upload(mxc_factor *F) {
         const bool use128 = n128 >= 2 * 256;
         auto edge = [&](size_t bi) {
             const UpdDesc &u = blocks[bi];
-            if (force && (*force)[bi] > 0) return (*force)[bi];
             if (use128 && wide128(u)) return 128;
             return (use16 && tiny16(u)) ? 16 : F->tune[kind_of(kind)][tile_bucket(u.M, u.N, u.K)];
         };
@@ -652,11 +636,6 @@ static int flatten_upload(mxc_factor *F) {
                                                    // factored by the previous step's trailing launch
         std::vector<int64_t> folded_s;             // ... and whose TRSM of this step it applied
         const size_t nst = F->blk_steps[l].size();
-        // second-stream updates merged into later trailing launches: per step, the
-        // column slices and their supernodes
-        std::vector<std::vector<UpdDesc>> merged(nst);
-        std::vector<std::vector<int64_t>> merged_s(nst);
-        auto edge_of = [&](const UpdDesc &u) { return F->tune[kind_of(L_TRAIL)][tile_bucket(u.M, u.N, u.K)]; };
         for (size_t t = 0; t < nst; t++) {
             const StepBlocks &sb = F->blk_steps[l][t];
             // blocks of at most TINY_DIAG columns: one lane each; at most 16: one
@@ -703,54 +682,6 @@ static int flatten_upload(mxc_factor *F) {
             // (a join only after a fork: the second stream must already be part of
             // the work, also inside a graph capture)
             if (sb.panel_end && level_forked) F->factor_launches.push_back(Launch{L_JOIN, 0, 0, 0});
-            bool fork_t2 = false;
-            if (!sb.trail2.empty()) {
-                // FP64: fold the update right of the next panel into the next panel's
-                // three trailing launches, one column slice each, where it runs beside
-                // their diagonal tails (under graph replay the second stream's branch
-                // ran after the main one).  Each slice takes its supernode's own
-                // trailing edge; every merged launch must stay within the tail limit.
-                bool merge = F->merge_t2 && F->precision == MXC_FP64 && t + 3 < nst;
-                std::vector<std::vector<UpdDesc>> add(3);
-                std::vector<std::vector<int64_t>> add_s(3);
-                for (size_t q = 0; merge && q < sb.trail2.size(); q++) {
-                    const UpdDesc &u = sb.trail2[q];
-                    const double M = u.M, tot = (double)u.N * M - (double)u.N * u.N / 2.0;
-                    int cut[4] = {0, 0, 0, u.N};
-                    for (int k = 1; k <= 2; k++) {      // area-balanced cuts on 64-column boundaries
-                        int a = cut[k - 1];
-                        while (a < u.N && ((double)a * M - (double)a * a / 2.0) < tot * k / 3.0) a += NB;
-                        cut[k] = std::min(a, u.N);
-                    }
-                    for (int k = 0; k < 3; k++) {
-                        if (cut[k + 1] <= cut[k]) continue;
-                        add[k].push_back(column_slice(u, cut[k], cut[k + 1]));
-                        add_s[k].push_back(sb.trail2_s[q]);
-                    }
-                }
-                for (int k = 0; merge && k < 3; k++) {
-                    const StepBlocks &tg = F->blk_steps[l][t + 1 + k];
-                    long long cnt[3] = {0, 0, 0};
-                    auto slot = [](int ts) { return ts == 32 ? 0 : ts == 64 ? 1 : 2; };
-                    for (const UpdDesc &u : tg.trail) cnt[slot(edge_of(u))] += lower_tiles(u, edge_of(u), true);
-                    for (size_t q = 0; q < add[k].size(); q++) {
-                        int e = 0;
-                        for (size_t r = 0; r < tg.trail.size(); r++)
-                            if (tg.trail_s[r] == add_s[k][q]) e = edge_of(tg.trail[r]);
-                        if (e == 0) { merge = false; break; }
-                        cnt[slot(e)] += lower_tiles(add[k][q], e, true);
-                    }
-                    for (int c = 0; merge && c < 3; c++) merge = cnt[c] <= PD_MAX_TILES_FP64;
-                }
-                if (merge) {
-                    for (int k = 0; k < 3; k++) {
-                        merged[t + 1 + k].insert(merged[t + 1 + k].end(), add[k].begin(), add[k].end());
-                        merged_s[t + 1 + k].insert(merged_s[t + 1 + k].end(), add_s[k].begin(), add_s[k].end());
-                    }
-                } else {
-                    fork_t2 = true;
-                }
-            }
             // the next step's diagonal blocks, one per trailing block, and (FP64)
             // whether its TRSM can be folded in: a full 64-column diagonal block
             // with rows below it, all inside this trailing block
@@ -771,28 +702,16 @@ static int flatten_upload(mxc_factor *F) {
                                   sb.trail[q].N >= NB && sb.trail[q].M == nx.trsm[rt].M + NB;
                 }
             }
-            if (merged[t].empty()) {
-                emit(L_TRAIL, sb.trail, true, &follow, &fused, nullptr, &foldable, &folded);
-            } else {
-                // this step's trailing blocks, then the merged slices at their
-                // supernodes' edges
-                std::vector<UpdDesc> blocks(sb.trail);
-                std::vector<int> force(sb.trail.size(), 0);
-                for (size_t q = 0; q < merged[t].size(); q++) {
-                    int e = 0;
-                    for (size_t r = 0; r < sb.trail.size(); r++)
-                        if (sb.trail_s[r] == merged_s[t][q]) e = edge_of(sb.trail[r]);
-                    blocks.push_back(merged[t][q]);
-                    force.push_back(e);
-                }
-                emit(L_TRAIL, blocks, true, &follow, &fused, &force, &foldable, &folded);
-            }
-            if (fork_t2) {
+            emit(L_TRAIL, sb.trail, true, &follow, &fused, &foldable, &folded);
+            if (!sb.trail2.empty()) {
                 // the second-stream update starts when this step's own trailing
                 // update has finished, together with the next diagonal block's
                 // factorization: that single workgroup then finds a CU before the
                 // second stream's tiles fill them all (started beside the trailing
-                // update, it waited for the whole second-stream launch to drain)
+                // update, it waited for the whole second-stream launch to drain).
+                // (Cut into slices that joined the next panel's trailing launches,
+                // it ran at the tail kernels' occupancy: 64^3 diffusion FP64 16.29 ms
+                // so, 16.16 ms on the second stream)
                 F->factor_launches.push_back(Launch{L_FORK, 0, 0, 0});
                 emit(L_TRAIL2, sb.trail2, true);
                 level_forked = true;
@@ -1086,7 +1005,7 @@ static int build_plan(mxc_factor *F, const mxc_symbolic *S, const int64_t *Ap, c
                         u.ls_off = (int)(S->Lpi[s] + c_lo);
                         u.ldc = (int)nsrow;
                         (part == 0 ? sb.trail : sb.trail2).push_back(u);
-                        (part == 0 ? sb.trail_s : sb.trail2_s).push_back(s);
+                        if (part == 0) sb.trail_s.push_back(s);
                         double n1 = (double)u.N, n3 = (double)(u.M - u.N), kk = (double)u.K;
                         F->flops_trail += kk * n1 * (n1 + 1) + 2.0 * n3 * n1 * kk;
                     }
@@ -1708,6 +1627,13 @@ static void launch_tile(mxc_factor *F, const Launch &L, T *W, hipStream_t st = n
         if (L.tile == 32) {
             hipLaunchKernelGGL((k_tile<T, MODE, 32>), g, dim3(64), 0, st, F->d_desc, F->d_tiles + L.begin, W,
                                F->d_Ls, Lh, adiag, pda);
+            return;
+        }
+    }
+    if constexpr (PD && std::is_same<T, double>::value) {
+        if (L.tile == 64 && F->fold_trsm) {
+            hipLaunchKernelGGL((k_tile<T, MODE, 64, PD, true>), g, dim3(256), 0, st, F->d_desc, F->d_tiles + L.begin,
+                               W, F->d_Ls, Lh, adiag, pda);
             return;
         }
     }
