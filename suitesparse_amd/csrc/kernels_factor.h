@@ -1010,7 +1010,8 @@ __device__ __forceinline__ int panel_elim(T (&a)[16], int nreal, T floor_l, bool
 // first failing column (-1 on entry), sfail[1] the breakdown flag (0 on entry).
 // The inverse's four diagonal blocks hold the identity on entry (potrf_init).
 // The caller synchronizes before; the block and its inverse are complete (and
-// visible) on return.
+// visible) on return.  Between two barriers no entry of LDS that one wave reads
+// or writes is written by another.
 template <typename T>
 __device__ __forceinline__ void potrf_init(T *S, int *sfail) {
     const int tid = threadIdx.x;
@@ -1055,13 +1056,13 @@ __device__ __forceinline__ void potrf_core(T *S, int *sfail, int nb, const doubl
                 for (int j = 0; j < p - 1; j++) inv_row(p - 1, j);
             __syncthreads();
         }
+        T a[16];
         if (wave < 2) {
             // wave 0: row R + lane (past the last row: that row again, not stored);
             // wave 1: the diagonal block's rows, then the inverse's identity rows
             const bool row = R + lane < NB;
             const T *ar = (wave == 0 || lane < 16) ? S + min(R + lane, NB - 1) * PS + R
                                                    : S + inv_at<T>(p, p) + (lane & 15) * PS;
-            T a[16];
 #pragma unroll
             for (int c = 0; c < 16; c++) a[c] = ar[c];
             T floor_l = 0;
@@ -1071,7 +1072,7 @@ __device__ __forceinline__ void potrf_core(T *S, int *sfail, int nb, const doubl
             if (wave == 0) {
                 if (lane == 0 && badj < 16 && sfail[0] < 0) sfail[0] = R + badj;
                 if (SAFE && lane == 0 && brk) sfail[1] = 1;
-                if (row) {
+                if (lane >= 16 && row) {
 #pragma unroll
                     for (int c = 0; c < 16; c++) S[(R + lane) * PS + R + c] = a[c];
                 }
@@ -1094,11 +1095,15 @@ __device__ __forceinline__ void potrf_core(T *S, int *sfail, int nb, const doubl
             }
         }
         __syncthreads();
+        // L(p, p), now that waves 0 and 1 have both read A(p, p); nothing before the
+        // last barrier reads it (wave 1 has it as wave 0 does, and less to do next)
+        if (wave == 1 && lane < 16) {
+#pragma unroll
+            for (int c = 0; c < 16; c++) S[(R + lane) * PS + R + c] = a[c];
+        }
     }
-    if (np > 1) {
-        if (wave < np - 1) inv_row(np - 1, wave);
-        __syncthreads();
-    }
+    if (wave < np - 1) inv_row(np - 1, wave);
+    __syncthreads();
 }
 
 // SAFE (rho > 0, low-precision factor): a pivot d_jj <= rho * a_jj (a_jj the

@@ -1,0 +1,63 @@
+// potrf_block on the CPU: the factor and the inverse of a diagonal block against
+// a plain Cholesky factorization, and bit for bit the same whichever wave is
+// first between two barriers.
+//
+//   diag_block fp64|fp32 nb
+#include "kernels_factor.h"
+
+using namespace mxc;
+
+template <typename T>
+static int check(int nb) {
+    const int ld = nb + 3;
+    const double tol = std::is_same<T, double>::value ? 1e-13 : 1e-4;
+    std::vector<double> A(nb * nb), L(nb * nb, 0.0), X(nb * nb, 0.0);
+    unsigned seed = 12345u + nb;
+    auto rnd = [&] { return (int)((seed = seed * 1664525u + 1013904223u) >> 8) / 8388608.0 - 1.0; };
+    for (int j = 0; j < nb; j++)
+        for (int i = j; i < nb; i++) A[i + j * nb] = (double)(T)(i == j ? 4.0 + rnd() : rnd() / sqrt((double)nb));
+    for (int j = 0; j < nb; j++)
+        for (int i = j; i < nb; i++) {
+            double s = A[i + j * nb];
+            for (int k = 0; k < j; k++) s -= L[i + k * nb] * L[j + k * nb];
+            L[i + j * nb] = i == j ? sqrt(s) : s / L[j + j * nb];
+        }
+    for (int c = 0; c < nb; c++)
+        for (int i = c; i < nb; i++) {
+            double s = i == c;
+            for (int k = c; k < i; k++) s -= L[i + k * nb] * X[k + c * nb];
+            X[i + c * nb] = s / L[i + i * nb];
+        }
+    std::vector<T> W0((size_t)ld * nb + nb * nb, (T)7), out[2];
+    for (int j = 0; j < nb; j++)
+        for (int i = j; i < nb; i++) W0[i + j * ld] = (T)A[i + j * nb];
+    const DiagTask t{0, (long long)ld * nb, ld, nb, 100, 0};
+    const int orders[2][4] = {{0, 1, 2, 3}, {3, 2, 1, 0}};
+    for (int o = 0; o < 2; o++) {
+        std::vector<T> W = W0, S(potrf_lds<T>(false) / sizeof(T));
+        int sfail[2], fail = INT_MAX;
+        emu::run(orders[o], [&] {
+            potrf_block<T, false>(t, W.data(), S.data(), sfail, &fail, (const double *)nullptr, 0.0, Redo{},
+                                  (double *)nullptr);
+        });
+        double err = 0;
+        for (int j = 0; j < nb; j++)
+            for (int i = j; i < nb; i++) {
+                err = max(err, fabs((double)W[i + j * ld] - L[i + j * nb]));
+                err = max(err, fabs((double)W[t.winv + i + j * nb] - X[i + j * nb]));
+            }
+        printf("first wave %d: error %.2e, fail %d\n", orders[o][0], err, fail);
+        if (!(err <= tol) || fail != INT_MAX) return 1;
+        out[o] = W;
+    }
+    if (memcmp(out[0].data(), out[1].data(), out[0].size() * sizeof(T))) {
+        printf("the result depends on the order of the waves\n");
+        return 1;
+    }
+    return 0;
+}
+
+int main(int argc, char **argv) {
+    if (argc != 3) return 2;
+    return !strcmp(argv[1], "fp64") ? check<double>(atoi(argv[2])) : check<float>(atoi(argv[2]));
+}
