@@ -970,18 +970,28 @@ __device__ __forceinline__ void store16(T *S, int r0, int c0, const typename Mfm
 // the inverse of the diagonal block.  Each pivot costs one reciprocal square
 // root (no divide on the serial path): L_jj = d_jj r_j and L_ij = a_ij r_j
 // with r_j = 1/sqrt(d_jj).  Returns the first non-positive pivot among the
-// panel's nreal real columns (16 if none), wave-uniform; from that column on
-// the values are not numbers.  SAFE: *brk is set when a pivot falls to its floor or below
-// (floor_l, lane j holds column j's: rho * a_jj, a_jj the assembled diagonal
-// of A): the block's result is then not used (redo_block64 refactors it).
-template <typename T, bool SAFE>
-__device__ __forceinline__ int panel_elim(T (&a)[16], int nreal, T floor_l, bool *brk) {
-    unsigned badm = 0, lowm = 0;    // bit j: pivot j is not positive / at or below its floor
+// panel's nreal real columns (16 if none), wave-uniform.  SAFE: *brk is set
+// when a pivot falls to its floor or below (floor_l, lane j holds column j's:
+// rho * a_jj, a_jj the assembled diagonal of A): the block's result is then not
+// used (redo_block64 refactors it).
+//
+// A non-positive pivot is replaced by 1, so that the values after it stay
+// finite.  The test would lie on the chain from pivot to pivot, so the columns
+// are eliminated without it first (REPLACE false: NaN from that pivot on), and
+// once more with it, from the entries entry(c) of the lane's row again, if a
+// pivot was not positive.
+template <typename T, bool SAFE, bool REPLACE>
+__device__ __forceinline__ void panel_pivots(T (&a)[16], T floor_l, int lane, unsigned &badm, unsigned &lowm) {
+    badm = lowm = 0;                // bit j: pivot j is not positive / at or below its floor
     T djj = lane_bcast(a[0], 0);
 #pragma unroll
     for (int j = 0; j < 16; j++) {
         badm |= (unsigned)__ballot(!(djj > (T)0)) & (1u << j);
         if (SAFE) lowm |= (unsigned)__ballot(djj <= lane_bcast(floor_l, j)) & (1u << j);
+        if (REPLACE && !(djj > (T)0)) {
+            djj = (T)1;
+            if (lane == j) a[j] = (T)1;
+        }
         const T l = a[j] * rsqrt_nr(djj);
         a[j] = l;
         if (j + 1 < 16) {
@@ -997,7 +1007,28 @@ __device__ __forceinline__ int panel_elim(T (&a)[16], int nreal, T floor_l, bool
 #pragma unroll
         for (int c = j + 2; c < 16; c++) a[c] -= l * bl[c];
     }
+}
+
+template <typename T, bool SAFE, typename Entry>
+__device__ __forceinline__ int panel_elim(T (&a)[16], Entry entry, int nreal, T floor_l, int lane, bool *brk) {
     const unsigned realm = nreal >= 16 ? 0xffffu : (1u << nreal) - 1;
+    unsigned badm, lowm;
+#pragma unroll
+    for (int c = 0; c < 16; c++) a[c] = entry(c);
+    panel_pivots<T, SAFE, false>(a, floor_l, lane, badm, lowm);
+    if (__builtin_expect((badm & realm) != 0, 0)) {
+        // (one load at a time, from addresses that the compiler takes for others than
+        // the first ones: it would keep those in registers throughout, 98 instead of
+        // 55 in k_potrf_small)
+        int o = 0;
+        asm volatile("" : "+v"(o));
+#pragma unroll
+        for (int c = 0; c < 16; c++) {
+            a[c] = entry(c + o);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        panel_pivots<T, SAFE, true>(a, floor_l, lane, badm, lowm);
+    }
     if (SAFE && (lowm & realm)) *brk = true;
     badm &= realm;
     return badm ? __builtin_ctz(badm) : 16;
@@ -1063,12 +1094,11 @@ __device__ __forceinline__ void potrf_core(T *S, int *sfail, int nb, const doubl
             const bool row = R + lane < NB;
             const T *ar = (wave == 0 || lane < 16) ? S + min(R + lane, NB - 1) * PS + R
                                                    : S + inv_at<T>(p, p) + (lane & 15) * PS;
-#pragma unroll
-            for (int c = 0; c < 16; c++) a[c] = ar[c];
+            auto entry = [&](int c) { return ar[c]; };
             T floor_l = 0;
             if (SAFE && lane < 16 && R + lane < nb) floor_l = (T)(rho * adiag[col0 + R + lane]);
             bool brk = false;
-            const int badj = panel_elim<T, SAFE>(a, nb - R, floor_l, &brk);
+            const int badj = panel_elim<T, SAFE>(a, entry, nb - R, floor_l, lane, &brk);
             if (wave == 0) {
                 if (lane == 0 && badj < 16 && sfail[0] < 0) sfail[0] = R + badj;
                 if (SAFE && lane == 0 && brk) sfail[1] = 1;
@@ -1186,16 +1216,15 @@ __global__ __launch_bounds__(256) void k_potrf_small(const DiagTask *__restrict_
     const int nb = t.nb;
     // lanes 0..15: the block's rows (extended by the identity), lanes 16..31: identity rows
     T a[16];
-#pragma unroll
-    for (int c = 0; c < 16; c++) {
+    auto entry = [&](int c) {
         // (loads from inside the block, unconditional: a predicated load is a branch each)
         const T v = W[t.off + min(lane, nb - 1) + (long long)min(c, nb - 1) * t.ld];
-        a[c] = (lane < nb && c <= lane) ? v : ((lane < 32 && (lane & 15) == c) ? (T)1 : (T)0);
-    }
+        return (lane < nb && c <= lane) ? v : ((lane < 32 && (lane & 15) == c) ? (T)1 : (T)0);
+    };
     T floor_l = 0;
     if (SAFE && lane < nb) floor_l = (T)(rho * adiag[t.col0 + lane]);
     bool brk = false;
-    const int badj = panel_elim<T, SAFE>(a, nb, floor_l, &brk);
+    const int badj = panel_elim<T, SAFE>(a, entry, nb, floor_l, lane, &brk);
     if (SAFE && brk) {
         // breakdown: leave the assembled block in W for the FP64 redo
         if (lane == 0) redo_push(rd, t);

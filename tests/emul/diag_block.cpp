@@ -1,14 +1,14 @@
 // potrf_block on the CPU: the factor and the inverse of a diagonal block against
-// a plain Cholesky factorization, and bit for bit the same whichever wave is
-// first between two barriers.
+// a plain Cholesky factorization (a non-positive pivot reported and replaced by
+// 1), and bit for bit the same whichever wave is first between two barriers.
 //
-//   diag_block fp64|fp32 nb
+//   diag_block fp64|fp32 nb [column whose diagonal entry is negative]
 #include "kernels_factor.h"
 
 using namespace mxc;
 
 template <typename T>
-static int check(int nb) {
+static int check(int nb, int bad) {
     const int ld = nb + 3;
     const double tol = std::is_same<T, double>::value ? 1e-13 : 1e-4;
     std::vector<double> A(nb * nb), L(nb * nb, 0.0), X(nb * nb, 0.0);
@@ -16,10 +16,16 @@ static int check(int nb) {
     auto rnd = [&] { return (int)((seed = seed * 1664525u + 1013904223u) >> 8) / 8388608.0 - 1.0; };
     for (int j = 0; j < nb; j++)
         for (int i = j; i < nb; i++) A[i + j * nb] = (double)(T)(i == j ? 4.0 + rnd() : rnd() / sqrt((double)nb));
+    if (bad >= 0) A[bad + bad * nb] = -1.0;
+    int first = INT_MAX;
     for (int j = 0; j < nb; j++)
         for (int i = j; i < nb; i++) {
             double s = A[i + j * nb];
             for (int k = 0; k < j; k++) s -= L[i + k * nb] * L[j + k * nb];
+            if (i == j && !(s > 0)) {
+                first = min(first, 100 + j);
+                s = 1.0;
+            }
             L[i + j * nb] = i == j ? sqrt(s) : s / L[j + j * nb];
         }
     for (int c = 0; c < nb; c++)
@@ -43,11 +49,12 @@ static int check(int nb) {
         double err = 0;
         for (int j = 0; j < nb; j++)
             for (int i = j; i < nb; i++) {
-                err = max(err, fabs((double)W[i + j * ld] - L[i + j * nb]));
-                err = max(err, fabs((double)W[t.winv + i + j * nb] - X[i + j * nb]));
+                const double e = max(fabs((double)W[i + j * ld] - L[i + j * nb]),
+                                     fabs((double)W[t.winv + i + j * nb] - X[i + j * nb]));
+                if (!(e <= err)) err = e;          // (a NaN stays)
             }
         printf("first wave %d: error %.2e, fail %d\n", orders[o][0], err, fail);
-        if (!(err <= tol) || fail != INT_MAX) return 1;
+        if (!(err <= tol) || fail != first) return 1;
         out[o] = W;
     }
     if (memcmp(out[0].data(), out[1].data(), out[0].size() * sizeof(T))) {
@@ -58,6 +65,7 @@ static int check(int nb) {
 }
 
 int main(int argc, char **argv) {
-    if (argc != 3) return 2;
-    return !strcmp(argv[1], "fp64") ? check<double>(atoi(argv[2])) : check<float>(atoi(argv[2]));
+    if (argc < 3) return 2;
+    const int nb = atoi(argv[2]), bad = argc > 3 ? atoi(argv[3]) : -1;
+    return !strcmp(argv[1], "fp64") ? check<double>(nb, bad) : check<float>(nb, bad);
 }

@@ -33,3 +33,12 @@ def program(tmp_path_factory):
 def test_factor_and_inverse_do_not_depend_on_wave_order(program, precision, nb):
     out = subprocess.run([program, precision, str(nb)], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stdout + out.stderr
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("nb,bad", [(9, 0), (16, 15), (37, 20), (64, 5), (64, 63)])
+def test_non_positive_pivot_is_replaced_by_one(program, precision, nb, bad):
+    """The factor and the inverse of a block with a negative diagonal entry stay
+    finite: the pivot is reported and 1 takes its place."""
+    out = subprocess.run([program, precision, str(nb), str(bad)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
