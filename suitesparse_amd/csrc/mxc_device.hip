@@ -2706,9 +2706,9 @@ extern "C" int mxc_set_option(mxc_factor *F, int option, int64_t value) {
             drop_factor_graph(F);
             return MXC_OK;
         case MXC_OPT_SPLIT16:
+            if (F->split16 == (value != 0)) return MXC_OK;
             F->split16 = value != 0;
-            drop_factor_graph(F);
-            return MXC_OK;
+            return flatten_upload(F);           // the tile edges of FP32 update launches depend on it
         case MXC_OPT_SOLVE_CHAIN:
             F->chain = value != 0;
             drop_sweep_graphs(F);
