@@ -366,7 +366,10 @@ int mxc_solve_refine_segments(mxc_factor *F, const double *B, int64_t nrhs, doub
  * bucket's blocks (reps launches each, HIP events), keeps the fastest, rebuilds
  * the plan and returns the table (3*75 entries, kind-major; may be NULL).  It
  * scribbles on the numeric factor: call it before mxc_factorize.
- * mxc_set_tiles installs a saved table; mxc_get_tiles reads the current one. */
+ * mxc_set_tiles installs a saved table; mxc_get_tiles reads the current one.
+ * With the default table (64, and 32 for blocks of at most 64 rows and 32
+ * columns) FP32 update launches also take tiles of 128 where these fill the
+ * device; any other table is taken as it is. */
 int mxc_autotune(mxc_factor *F, int reps, int *table);
 int mxc_set_tiles(mxc_factor *F, const int *table);
 int mxc_get_tiles(const mxc_factor *F, int *table);

@@ -142,6 +142,11 @@ static inline int tile_bucket(int M, int N, int K) {
 }
 static constexpr int NBUCKET = 75;
 static constexpr int NKIND = 3;     // 0 descendant update, 1 trailing, 2 TRSM
+// default tile edge: 32 up to 64 x 32, else 64
+static inline int default_tile(int bucket) {
+    const int mb = bucket / 15, nb = (bucket / 3) % 5;
+    return mb <= 2 && nb <= 2 ? 32 : 64;
+}
 static inline int kind_of(int launch_kind) {
     return launch_kind == 0 ? 0 : (launch_kind == 3 || launch_kind == 9 || launch_kind == 14) ? 1 : 2;
 }
@@ -309,10 +314,8 @@ struct mxc_factor {
     std::vector<std::vector<StepBlocks>> blk_steps;   // per level, per 64-column step
     size_t plan_bytes = 0;                            // bytes of d_desc + d_tiles + d_diag + d_small
 
-    // tile edge per (M, N) bucket: 32 up to 64 x 32, 128 for M > 128 and N > 32,
-    // else 64 (mxc_set_tile overrides an entry before the plan is built)
+    // tile edge per (M, N, K) bucket: default_tile, unless set or tuned by the caller
     int tune[NKIND][NBUCKET];
-    bool tiles_default = true;             // no table set or tuned by the caller
 
     // hipGraph replay: the launch sequence depends only on the pattern, so it is
     // captured once and replayed for every refactorization / solve
@@ -467,6 +470,9 @@ static int flatten_upload(mxc_factor *F) {
         return (int64_t)(std::upper_bound(F->Super.begin(), F->Super.end(), (int64_t)base) - F->Super.begin()) - 1;
     };
     F->nsmall = 0;
+    bool default_table = true;
+    for (int k = 0; k < NKIND; k++)
+        for (int b = 0; b < NBUCKET; b++) default_table = default_table && F->tune[k][b] == default_tile(b);
     // follow[i] (trailing blocks): the next step's diagonal task of block i's
     // supernode, or null.  A block tiled at 64 or 128 gets it as its tail (pd);
     // fused[i] records that, so the next step's diagonal launch skips it.
@@ -492,14 +498,14 @@ static int flatten_upload(mxc_factor *F) {
         // split-FP16 tiles (half the operand bytes per product) where they make at least
         // two workgroups per CU; a level with fewer leaves CUs idle with them (41^3 FP32
         // factor 2.27 ms with 64-wide tiles throughout, 2.37 ms with 128; 80^3 27-point
-        // 26.9 and 25.2 ms).  FP64 tiles of 128 were slower in both.  A table that the
-        // caller set or tuned is taken as it is.
+        // 26.9 and 25.2 ms).  FP64 tiles of 128 were slower in both.  A table other than
+        // the default one is taken as it is.
+        const bool may128 = F->precision != MXC_FP64 && F->split16 && kind == L_UPD && default_table;
         auto wide128 = [&](const UpdDesc &u) {
-            return F->precision != MXC_FP64 && F->split16 && F->tiles_default && kind == L_UPD && u.M > 128 &&
-                   u.N > 64 && u.K > 32;
+            return may128 && u.M > 128 && u.N > 64 && u.K > 32;
         };
         long long n128 = 0;
-        if (F->precision != MXC_FP64 && F->tiles_default && kind == L_UPD)
+        if (may128)
             for (const UpdDesc &u : blocks) n128 += wide128(u) ? lower_tiles(u, 128, lower_only) : 0;
         const bool use128 = n128 >= 2 * 256;
         auto edge = [&](size_t bi) {
@@ -1347,10 +1353,7 @@ extern "C" int mxc_factor_create_in(const mxc_symbolic *S, const int64_t *Ap, co
     F->precision = precision;
     F->rho = precision == MXC_FP32 ? 1e-6 : 0.0;
     for (int k = 0; k < NKIND; k++)
-        for (int b = 0; b < NBUCKET; b++) {
-            int mb = b / 15, nbk = (b / 3) % 5;
-            F->tune[k][b] = (mb <= 2 && nbk <= 2) ? 32 : 64;
-        }
+        for (int b = 0; b < NBUCKET; b++) F->tune[k][b] = default_tile(b);
     hipError_t e = hipSetDevice(g_device);
     {
         std::lock_guard<std::recursive_mutex> lk(g_rt_mutex);
@@ -2654,7 +2657,6 @@ static int autotune_impl(mxc_factor *F, int reps, int *table) {
             F->tune[kind][b] = best_ts;
         }
     }
-    F->tiles_default = false;
     F->values_loaded = false;        // the timing launches scribbled on L
     int rc = flatten_upload(F);
     if (rc) return rc;
@@ -2678,7 +2680,6 @@ extern "C" int mxc_set_tiles(mxc_factor *F, const int *table) {
         if (table[q] != 32 && table[q] != 64 && table[q] != 128) return MXC_INVALID;
     for (int k = 0; k < NKIND; k++)
         for (int b = 0; b < NBUCKET; b++) F->tune[k][b] = table[k * NBUCKET + b];
-    F->tiles_default = false;
     return flatten_upload(F);
 }
 

@@ -96,6 +96,19 @@ def test_a_setting_of_split16_sets_the_tiles(gpu):
     _check_factor(A, cm, L, blocks, 1e-4)
 
 
+def test_a_table_read_back_and_set_leaves_the_plan(gpu):
+    """The default table means the default rules, set or not; another table is
+    taken as it is."""
+    A, cm, L, _ = _analyzed("fp32")
+    table = L.tiles()
+    L.set_tiles(table)
+    assert L.tiles() == table and L.info()["update_tiles"] == TILES_128
+    L.set_tiles([64] * len(table))
+    assert L.info()["update_tiles"] == TILES_64
+    L.set_tiles(table)
+    assert L.info()["update_tiles"] == TILES_128
+
+
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
 def test_wide_launches(gpu, prec):
     """A 27-point 64^3 system end to end: the residual of a solve, against n u with
