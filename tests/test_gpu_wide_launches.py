@@ -1,13 +1,16 @@
-"""GPU: factors whose launches are wide enough for the rules on tile counts.
+"""GPU: factors whose launches are wide enough for the rules on tile counts, and
+that those rules were taken.
 
 Forty dense blocks of 192 columns, all coupled to a separator of 650 (which the
 last block joins in one supernode of 842 columns): 39 update blocks of 650 x 650
 into one target, and 39 supernodes of 842 rows whose trailing updates share a
 launch.  Of edge 128 an update block has 21 tiles in its lower part, 819 in all,
-of edge 64 it has 66.  The factor is compared entry by entry with one formed
+of edge 64 it has 66; the first trailing launch, of 39 blocks of 778 x 128, has
+39 * 25 = 975 tiles of 64.  The factor is compared entry by entry with one formed
 block by block in FP64 on the host: in FP32 the 39 subtractions from diagonal
 entries of 84 stay within 39 u 84 = 2e-4, 3e-5 of max |L| = 6.6; 1e-4 and, with
-u = 1.1e-16, 1e-12 are asked for.
+u = 1.1e-16, 1e-12 are asked for.  A 128-wide tile left out of one block's
+update changes L by 80 times 1e-4 or more, as the oracle shows.
 """
 import numpy as np
 import pytest
@@ -107,6 +110,30 @@ def test_a_table_read_back_and_set_leaves_the_plan(gpu):
     assert L.info()["update_tiles"] == TILES_64
     L.set_tiles(table)
     assert L.info()["update_tiles"] == TILES_128
+
+
+def _launches(L):
+    """Update, diagonal, TRSM and trailing launches of the plan."""
+    counts, ms = np.zeros(8, dtype=np.int64), np.zeros(4)
+    _lib.check("mxc_factor_stats", _lib.lib().mxc_factor_stats(L._num, cholmod._ptr(counts), cholmod._ptr(ms)))
+    return counts[:4].tolist()
+
+
+def test_fp32_update_launch_of_128_wide_tiles(gpu):
+    A, cm, L, blocks = _analyzed("fp32")
+    assert L.info()["update_tiles"] == TILES_128
+    Lref = _check_factor(A, cm, L, blocks, 1e-4)
+    for lost in [(0, 0, 0), (5, 256, 128), (38, 512, 0), (20, 384, 384)]:
+        assert np.abs(_factor(*blocks, lost) - Lref).max() > 50 * 1e-4 * np.abs(Lref).max()
+
+
+def test_fp64_tails_in_a_launch_of_975_tiles(gpu):
+    """The diagonal blocks of steps 1 and 2 are the tails of the trailing launches
+    of 975 and 468 tiles, those of the 842 columns above tails too, except for the
+    last one, whose trailing block is below 64 columns: three diagonal launches."""
+    A, cm, L, blocks = _analyzed("fp64")
+    assert _launches(L)[1] == 3
+    _check_factor(A, cm, L, blocks, 1e-12)
 
 
 @pytest.mark.parametrize("prec", ["fp64", "fp32"])
