@@ -27,6 +27,13 @@ pytestmark = pytest.mark.gpu
 SPD = ["bcsstk01.tri", "bcsstk02.tri", "can___24.mtx", "k01up", "r5lo", "diag", "two.tri", "2diag.tri"]
 
 
+@pytest.fixture(autouse=True)
+def _host_cholmod(ref_lib):
+    """The caller links the host CHOLMOD: without the reference there is nothing to
+    build it from (the fixture skips); with it, it must be there."""
+    assert FLOW.exists(), "tests/dropin/_build/dropin_flow not built"
+
+
 def _check(v, supernodal_expected=None):
     assert v["gpu_status"] == v["host_status"], (v["gpu_status"], v["host_status"])
     assert v["gpu_minor"] == v["host_minor"]
@@ -73,7 +80,6 @@ def _check(v, supernodal_expected=None):
 @pytest.mark.parametrize("mode", ["supernodal", "auto"])
 @pytest.mark.parametrize("name", SPD)
 def test_demo_flow_through_dropin(gpu, name, mode):
-    assert FLOW.exists(), "tests/dropin/_build/dropin_flow not built"
     print(f"case {name} {mode}", flush=True)
     out, v = run_flow(FIX / name, *(["supernodal"] if mode == "supernodal" else []))
     print(out.stdout[-1500:], flush=True)
