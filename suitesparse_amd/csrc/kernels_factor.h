@@ -300,7 +300,7 @@ __device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W
 //
 // With a folded TRSM (UpdDesc::fold) the tail publishes the factored block:
 // ready[pd] is set once its L and inverse are in W (a device-scope release
-// after the workgroup's stores), and the tiles of column 0 below it wait for
+// of every wave after its stores), and the tiles of column 0 below it wait for
 // that flag (device-scope acquire) before applying the inverse.  Producer
 // tiles come first in the launch (the first nfirst workgroups map to tiles
 // 0 .. nfirst-1, which hold them) and never wait, and workgroups start in
@@ -334,7 +334,10 @@ __device__ __forceinline__ void pd_tail(const PdArgs &pda, int pd, T *__restrict
         potrf_block<T, false, LOADED>(pda.diags[pd], W, S, sfail, pda.fail, adiag, pda.rho, pda.rd, nullptr);
     }
     if (publish) {
-        __syncthreads();                    // every wave's stores of L and the inverse are issued
+        // every wave waits for its own stores of L and the inverse: the release of the
+        // flag's store orders those of thread 0's wave only
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        __syncthreads();
         if (threadIdx.x == 0) __hip_atomic_store(pda.ready + pd, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     }
 }

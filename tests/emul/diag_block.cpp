@@ -3,6 +3,7 @@
 // 1), and bit for bit the same whichever wave is first between two barriers.
 //
 //   diag_block fp64|fp32 nb [column whose diagonal entry is negative]
+//   diag_block publish       a tail that publishes its block to other workgroups
 #include "kernels_factor.h"
 
 using namespace mxc;
@@ -64,7 +65,23 @@ static int check(int nb, int bad) {
     return 0;
 }
 
+static int publish() {
+    const int nb = NB;
+    std::vector<double> W(2 * nb * nb, 0.0);
+    for (int i = 0; i < nb; i++) W[i + i * nb] = 4.0;
+    const DiagTask t{0, nb * nb, nb, nb, 0, 0};
+    int fail = INT_MAX, ready = 0, abort = 0;
+    const PdArgs pda{&t, &fail, 0.0, Redo{}, &ready, &abort, 1};
+    std::vector<double> smem(potrf_lds<double>(false) / sizeof(double));
+    emu::run({0, 1, 2, 3}, [&] {
+        pd_tail<double, false>(pda, 0, W.data(), (unsigned char *)smem.data(), (const double *)nullptr, true);
+    });
+    printf("flag %d, lanes whose stores were not released before it: %d\n", ready, emu::unreleased_flags);
+    return ready == 1 && emu::unreleased_flags == 0 && W[0] == 2.0 && W[nb * nb] == 0.5 ? 0 : 1;
+}
+
 int main(int argc, char **argv) {
+    if (argc == 2 && !strcmp(argv[1], "publish")) return publish();
     if (argc < 3) return 2;
     const int nb = atoi(argv[2]), bad = argc > 3 ? atoi(argv[3]) : -1;
     return !strcmp(argv[1], "fp64") ? check<double>(nb, bad) : check<float>(nb, bad);

@@ -45,6 +45,7 @@ struct Lane {
     std::vector<char> stack;
     State state;
     unsigned ops;                         // cross-lane operations so far: which exchange buffer is in use
+    bool released;                        // a device-scope release since the last cross-lane operation
 };
 
 inline Lane lanes[THREADS];
@@ -67,6 +68,7 @@ inline void entry() {
 
 // every lane's (a, b), once all 64 have come here
 inline const Slot *exchange(double a, double b = 0) {
+    lanes[cur].released = false;
     const int w = cur >> 6, l = cur & 63, q = lanes[cur].ops++ & 1;
     slots[w][q][l] = Slot{a, b};
     yield(WAVE);
@@ -81,6 +83,7 @@ inline void run(const int (&order)[THREADS / 64], const std::function<void()> &f
         L.stack.resize(256 << 10);
         L.state = RUN;
         L.ops = 0;
+        L.released = false;
         getcontext(&L.ctx);
         L.ctx.uc_stack.ss_sp = L.stack.data();
         L.ctx.uc_stack.ss_size = L.stack.size();
@@ -113,6 +116,22 @@ inline void run(const int (&order)[THREADS / 64], const std::function<void()> &f
         if (lanes[0].state == DONE) return;
         for (Lane &L : lanes) L.state = RUN;
     }
+}
+
+// A release at a barrier or by one wave orders that wave's own stores only: a
+// flag that says to other workgroups that this one's stores are done needs a
+// device-scope release of every wave before it.
+inline int unreleased_flags = 0;          // flags stored while a lane had none
+
+inline void fence(int order, const char *scope) {
+    if (order == __ATOMIC_RELEASE && !strcmp(scope, "agent")) lanes[cur].released = true;
+}
+
+template <typename T>
+void atomic_store(T *p, T v, int order, int scope) {
+    if (scope == 1 && order == __ATOMIC_RELEASE)
+        for (const Lane &L : lanes) unreleased_flags += !L.released;
+    *p = v;
 }
 
 inline int readlane(int v, int k) { return (int)exchange(v)[k].a; }
@@ -151,7 +170,7 @@ V not_emulated(H, H, V c) {
 #define __builtin_amdgcn_readlane(v, k) emu::readlane(v, k)
 #define __builtin_amdgcn_readfirstlane(v) emu::readlane(v, 0)
 #define __builtin_amdgcn_wave_barrier() (void)emu::exchange(0)
-#define __builtin_amdgcn_fence(...)
+#define __builtin_amdgcn_fence(order, scope) emu::fence(order, scope)
 #define __builtin_amdgcn_sched_barrier(x)
 #define __builtin_amdgcn_s_setprio(x)
 #define __builtin_amdgcn_s_sleep(x)
@@ -160,9 +179,9 @@ V not_emulated(H, H, V c) {
 #define __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, x, y, z) emu::mfma16x16x4<double>(a, b, c)
 #define __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, x, y, z) emu::mfma16x16x4<float>(a, b, c)
 #define __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, x, y, z) emu::not_emulated(a, b, c)
-#define __HIP_MEMORY_SCOPE_AGENT 0
+#define __HIP_MEMORY_SCOPE_AGENT 1
 #define __HIP_MEMORY_SCOPE_WORKGROUP 0
-#define __hip_atomic_store(p, v, order, scope) (void)(*(p) = (v))
+#define __hip_atomic_store(p, v, order, scope) emu::atomic_store(p, v, order, scope)
 #define __hip_atomic_load(p, order, scope) (*(p))
 #define __hip_atomic_fetch_add(p, v, order, scope) (*(p) += (v))
 

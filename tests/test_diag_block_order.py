@@ -42,3 +42,10 @@ def test_non_positive_pivot_is_replaced_by_one(program, precision, nb, bad):
     finite: the pivot is reported and 1 takes its place."""
     out = subprocess.run([program, precision, str(nb), str(bad)], capture_output=True, text=True, timeout=300)
     assert out.returncode == 0, out.stdout + out.stderr
+
+
+def test_published_block_is_released_by_every_wave(program):
+    """The flag of a folding tail says that the block's L and inverse are in memory
+    for workgroups on other CUs: every wave has released its own stores before it."""
+    out = subprocess.run([program, "publish"], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, out.stdout + out.stderr
