@@ -664,7 +664,6 @@ __global__ __launch_bounds__(256, 1) void k_tile_grid(const UpdDesc *__restrict_
 }
 
 // ---------------------------------------------------------------------------
-// ---------------------------------------------------------------------------
 // FP32 factor, split-FP16 products (update and trailing blocks).  An FP32
 // value v of L in global row g is scaled by 2^s_g, s_g = 13 - floor(log2
 // sqrt(a_gg)) with a_gg the assembled diagonal of A (|L_gk| <= sqrt(a_gg), so
@@ -889,7 +888,7 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
 //   waves 2, 3, beside them: panel p-1's other updates (MFMA) and the sums
 //           T_pj = sum_k L_pk X_kj of the inverse's block row p
 //   then, all waves: the update of block column p+1 by panel p (MFMA) and
-//           X_pj = -X_pp T_pj
+//           X_pj = -X_pp T_pj; wave 1 stores L_pp, which both had to read
 // Two barriers per panel.  The lower factor is written back in place (the
 // strict upper triangle is left alone, as dpotrf leaves it) and inv(L) (zero
 // above the diagonal) goes to the block's inverse slot (ld nb).  A
@@ -897,9 +896,9 @@ __global__ __launch_bounds__(256, 2) void k_tile_h(const UpdDesc *__restrict__ d
 // ---------------------------------------------------------------------------
 
 // 1/sqrt(x) for x > 0: the hardware estimate y0 (relative error below 2^-23)
-// refined once to third order, y = y0 (1 + e/2 + 3e^2/8) with e = 1 - x y0^2:
-// the remaining term is below 2^-69, and the chain is four dependent
-// operations where two Newton steps take six (every pivot waits for it).
+// refined once to third order, y = y0 (1 + e/2 + 3e^2/8) with e = 1 - x y0^2
+// below 2^-22: the remaining term 5e^3/16 is below 2^-67, and the chain is four
+// dependent operations where two Newton steps take six (every pivot waits for it).
 __device__ __forceinline__ double rsqrt_nr(double x) {
     const double y = __builtin_amdgcn_rsq(x);
     const double e = fma(-x * y, y, 1.0);
@@ -1142,8 +1141,8 @@ __device__ __forceinline__ void potrf_core(T *S, int *sfail, int nb, const doubl
 // SAFE (rho > 0, low-precision factor): a pivot d_jj <= rho * a_jj (a_jj the
 // assembled diagonal of A) signals breakdown of the block.  Its low-precision
 // result is dropped and the same workgroup refactors the block in FP64 in
-// place (redo_block64, in the LDS of S and X), before anything reads it.  Without SAFE a pivot
-// <= 0 is reported as the failing column.
+// place (redo_block64, in the LDS of the block and its inverse), before anything
+// reads it.  Without SAFE a pivot <= 0 is reported as the failing column.
 //
 // potrf_block: the whole workgroup (256 threads) factors diagonal block t in
 // LDS (S: potrf_lds<T>(SAFE) bytes, potrf_core's layout;
@@ -1176,7 +1175,7 @@ __device__ __forceinline__ void potrf_block(const DiagTask &t, T *__restrict__ W
     __syncthreads();
     potrf_core<T, SAFE>(S, sfail, nb, adiag, t.col0, rho);
     if (SAFE && sfail[1]) {
-        // breakdown: the block again from W, in FP64, in the LDS of S and X
+        // breakdown: the block again from W, in FP64, in the same LDS
         redo_block64<T>(t, W, reinterpret_cast<double *>(S), tmp, sfail, tid, 256, rd, fail,
                         [] { __syncthreads(); });
         return;

@@ -838,7 +838,8 @@ __device__ __forceinline__ T lane_get(T v, int l) {
 // acc[z] += sum_j l[j] q[z / 4](j + 16 (z % 4)), q(m) = lane m's value of q (wave-uniform)
 template <typename T, int ZC, int NQ>
 __device__ __forceinline__ void fma_bcast(T (&acc)[ZC], const T (&l)[16], const T (&q)[NQ]) {
-    // four columns at a time (all the broadcasts at once spill scalar registers)
+    // four columns at a time: fewer broadcasts wait in scalar registers (which the
+    // wide backward sweeps spill all the same: 476 in k_chain_bwd<double, 8>)
 #pragma unroll
     for (int j0 = 0; j0 < 16; j0 += 4) {
 #pragma unroll

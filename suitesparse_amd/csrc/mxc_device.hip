@@ -443,6 +443,16 @@ static long long lower_tiles(const UpdDesc &u, int ts, bool lower_only) {
     return lower_only ? mt * nt - nt * (nt - 1) / 2 : mt * nt;
 }
 
+// CUs of the current device (queried once; plans are built by several threads)
+static int device_cus() {
+    static const int cus = [] {
+        int v = 0;
+        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, g_device) != hipSuccess || v <= 0) v = 256;
+        return v;
+    }();
+    return cus;
+}
+
 static int flatten_upload(mxc_factor *F) {
     std::vector<UpdDesc> descs;
     std::vector<Tile> tiles;
@@ -494,9 +504,9 @@ static int flatten_upload(mxc_factor *F) {
         long long n16 = 0;
         for (const UpdDesc &u : blocks) n16 += tiny16(u) ? 1 : 0;
         const bool use16 = n16 >= 200000;
-        // FP32 descendant updates of more than 128 rows and 64 columns take 128-wide
-        // split-FP16 tiles (half the operand bytes per product) where they make at least
-        // two workgroups per CU; a level with fewer leaves CUs idle with them (41^3 FP32
+        // FP32 descendant updates of more than 128 rows, 64 columns and one chunk of K take
+        // 128-wide split-FP16 tiles (half the operand bytes per product) where they make at
+        // least two workgroups per CU; a level with fewer leaves CUs idle with them (41^3 FP32
         // factor 2.27 ms with 64-wide tiles throughout, 2.37 ms with 128; 80^3 27-point
         // 26.9 and 25.2 ms).  FP64 tiles of 128 were slower in both.  A table other than
         // the default one is taken as it is.
@@ -507,7 +517,7 @@ static int flatten_upload(mxc_factor *F) {
         long long n128 = 0;
         if (may128)
             for (const UpdDesc &u : blocks) n128 += wide128(u) ? lower_tiles(u, 128, lower_only) : 0;
-        const bool use128 = n128 >= 2 * 256;
+        const bool use128 = n128 >= 2LL * device_cus();
         auto edge = [&](size_t bi) {
             const UpdDesc &u = blocks[bi];
             if (use128 && wide128(u)) return 128;
@@ -516,8 +526,9 @@ static int flatten_upload(mxc_factor *F) {
         long long total = 0;
         for (int ts : {16, 32, 64, 128}) {
             long long b = (long long)tiles.size();
-            // tails only in launches that fit on the device at once (a tail's
-            // kernel runs at lower occupancy)
+            // tails only up to a measured number of tiles (a tail's kernel runs at
+            // lower occupancy).  Such a launch need not fit on the device at once: the
+            // waits of a folded TRSM end because producer tiles are dispatched first
             bool allow = follow != nullptr && ts >= 64;
             if (allow) {
                 long long cnt = 0;
@@ -1575,17 +1586,6 @@ static inline Redo redo_args(const mxc_factor *F) {
     return Redo{F->d_fail + 1, F->d_redo, (const long long *)F->d_rowptr, (const int *)F->d_col,
                 (const double *)F->d_vals, (const long long *)F->d_perm, (const int *)F->d_pinv,
                 (const double *)F->d_beta};
-}
-
-// CUs of the current device (queried once)
-static int device_cus() {
-    static int cus = 0;
-    if (cus == 0) {
-        int v = 0;
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, g_device) != hipSuccess || v <= 0) v = 256;
-        cus = v;
-    }
-    return cus;
 }
 
 template <typename T, int MODE, bool PD = false>
